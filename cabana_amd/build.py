@@ -62,7 +62,7 @@ def build_library(verbose=False):
     # Per-particle kernels for Spline<0> .. Spline<6>; cell-tiled kernels for
     # orders 1 to 3.
     for order in range(7):
-        for src in ("ca_kernels", "ca_tiled") if 1 <= order <= 3 else ("ca_kernels",):
+        for src in ("ca_kernels", "ca_tiled", "ca_scatter") if 1 <= order <= 3 else ("ca_kernels",):
             obj = os.path.join(BUILD, "%s_o%d.o" % (src, order))
             jobs.append([hipcc] + COMMON + ["-DCA_ORDER=%d" % order, "-c",
                                             os.path.join(CSRC, src + ".hip"), "-o", obj])

@@ -683,18 +683,12 @@ struct TileShape
 {
     int T[3];
     int cap;
-    int max_tasks;
 };
 
-int base_cells( const int T[3], int order )
-{
-    const int spread = ( order == 2 ) ? 1 : 0;
-    return ( T[0] + spread ) * ( T[1] + spread ) * ( T[2] + spread );
-}
-
-// LDS bytes of the tiled kernels; mirrors their in-kernel layout.
-size_t tile_lds_bytes( TileKind kind, bool fp64, const int* slot_ng, int nslot,
-                       int rec_len, int order, const TileShape& sh )
+// LDS bytes of the tiled kernels; mirrors their in-kernel layout.  vals: the
+// values of a scatter record's slot.
+size_t tile_lds_bytes( TileKind kind, bool fp64, const int* slot_ng, int nslot, int vals,
+                       int order, const TileShape& sh )
 {
     const int extra = ( order == 1 ) ? 1 : 3;
     const size_t wn = (size_t)( sh.T[0] + extra ) * ( sh.T[1] + extra ) * ( sh.T[2] + extra );
@@ -712,101 +706,81 @@ size_t tile_lds_bytes( TileKind kind, bool fp64, const int* slot_ng, int nslot,
     int dt = 0;
     for ( int i = 0; i < nslot; ++i )
         dt += slot_ng[i];
-    const size_t nbase = (size_t)base_cells( sh.T, order );
-    const size_t rs = (size_t)record_stride( rec_len, (int)real );
     b = a16( 8 * (size_t)dt * wn );
-    b = a16( b + 4 * ( nbase + 1 ) );
-    b = a16( b + 4 * (size_t)sh.max_tasks ); // sorted task table
-    b = a16( b + 4 * (size_t)sh.max_tasks ); // unsorted tasks
-    b = a16( b + 4 * (size_t)sh.max_tasks ); // their length bucket and rank
-    b = a16( b + 4 * 2 * SCATTER_TASK_MAX ); // length histogram and offsets
-    b = a16( b + 2 * (size_t)sh.cap );
-    b = a16( b + real * rs * (size_t)sh.cap );
-    for ( int buf = 0; buf < 2; ++buf )
-    {
-        b = a16( b + 8 * runs );
-        b = a16( b + 4 * ( runs + 1 ) );
-    }
-    b = a16( b + 8 * 128 ); // part-table entries
-    b += 4 * 16 + 16;       // per-wave scan sums of a workgroup of up to 1024 threads
+    b = a16( b + real * ( SCATTER_BLOCK / 64 ) * ( scatter_sub( scatter_row( vals ) ) + 3 ) *
+                     scatter_record( fp64, scatter_row( vals ) ) );
+    b = a16( b + 8 * runs );
+    b = a16( b + 4 * ( runs + 1 ) );
     return b;
 }
 
 // Brick shape and part capacity.  Gathers use the largest cubic brick whose
 // windows fit 52 KB of LDS for FP32 (three workgroups per CU) and 78 KB for
-// FP64 (whose registers allow two), with parts of ~1.25x the mean brick
-// population.  Scatters sort a whole part in LDS: the brick is the largest
-// near-cubic one whose expected population (x1.2) fits a part (at most two
-// particles per thread) that, with the FP64 window, stays within 78 KB of
-// LDS (two workgroups per CU run at once, the kernel's register budget);
-// denser bricks are cut into several parts.
-bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int rec_len,
-                   int order, double mean_ppc, TileShape& out )
+// FP64 (whose registers allow two) and that leaves a workgroup for every CU
+// twice over where the mesh has the cells for it, with parts of ~1.25x the
+// mean brick population.
+bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int vals,
+                   int order, const int num_cell[3], double mean_ppc, TileShape& out )
 {
+    auto bricks_of = [&]( const TileShape& sh ) {
+        double n = 1.0;
+        for ( int d = 0; d < 3; ++d )
+            n *= ( num_cell[d] + sh.T[d] - 1 ) / sh.T[d];
+        return n;
+    };
     if ( kind == TILE_GATHER )
     {
-        static const int cand[] = { 8, 7, 6, 5, 4, 3, 2 };
-        for ( int c : cand )
+        bool found = false;
+        for ( int c = 8; c >= 2; --c )
         {
-            TileShape sh = { { c, c, c }, 0, 0 };
-            if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, rec_len, order, sh ) <=
-                 ( fp64 ? 78 : 52 ) * 1024 )
-            {
-                const double mean = mean_ppc * c * c * c;
-                double cap = 1.25 * mean;
-                cap = cap < 4096 ? 4096 : ( cap > ( 1 << 20 ) ? ( 1 << 20 ) : cap );
-                sh.cap = ( (int)cap + 255 ) / 256 * 256;
-                out = sh;
-                return true;
-            }
-        }
-        return false;
-    }
-    const size_t budget = 78 * 1024;
-    auto with_cap = [&]( TileShape sh, int cap ) {
-        sh.cap = cap;
-        sh.max_tasks = base_cells( sh.T, order ) + cap / SCATTER_TASK_MAX + 1;
-        return sh;
-    };
-    bool found = false;
-    TileShape best = {};
-    int best_vol = 0;
-    for ( int a = 2; a <= 8; ++a )
-        for ( int b = a; b <= a + 1 && b <= 8; ++b )
-            for ( int c = b; c <= b + 1 && c <= 8; ++c )
-            {
-                const int vol = a * b * c;
-                if ( vol <= best_vol )
-                    continue;
-                int cap = (int)( 1.2 * mean_ppc * vol ) + 32;
-                cap = ( cap + 63 ) / 64 * 64;
-                cap = cap < 256 ? 256 : cap;
-                if ( cap > scatter_cap_max( fp64 ) )
-                    continue;
-                TileShape sh = with_cap( { { a, b, c }, 0, 0 }, cap );
-                if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, rec_len, order, sh ) <=
-                     budget )
-                {
-                    best = sh;
-                    best_vol = vol;
-                    found = true;
-                }
-            }
-    if ( !found )
-    {
-        // Dense: the smallest brick with the largest part that fits.
-        for ( int cap = scatter_cap_max( fp64 ); cap >= 64; cap -= 64 )
-        {
-            TileShape sh = with_cap( { { 2, 2, 2 }, 0, 0 }, cap );
-            if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, rec_len, order, sh ) <= budget )
-            {
-                best = sh;
-                found = true;
+            TileShape sh = { { c, c, c }, 0 };
+            if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, vals, order, sh ) >
+                 (size_t)( fp64 ? 78 : 52 ) * 1024 )
+                continue;
+            const double mean = mean_ppc * c * c * c;
+            double cap = 1.25 * mean;
+            cap = cap < 1024 ? 1024 : ( cap > ( 1 << 20 ) ? ( 1 << 20 ) : cap );
+            sh.cap = ( (int)cap + 255 ) / 256 * 256;
+            out = sh;
+            found = true;
+            if ( bricks_of( sh ) >= 512.0 || mean < 256.0 )
                 break;
-            }
         }
+        return found;
     }
-    out = best;
+    // Scatters: the brick with the most cells per window node (fewest grid
+    // atomics per cell) whose LDS lets a full set of workgroups run on a CU,
+    // among those that give every CU several bricks.  Above 2^20 bricks, where
+    // the part table itself is large, two workgroups per CU.
+    const int extra = ( order == 1 ) ? 1 : 3;
+    const int c = scatter_cells_k( order );
+    const int waves = scatter_waves( fp64, scatter_row( vals ) );
+    bool found = false;
+    double best_bricks = 0.0;
+    for ( int w = waves; w >= 2 && ( !found || best_bricks > 1048576.0 ); w = w > 2 ? 2 : 1 )
+    {
+        double best = -1.0;
+        for ( int a = 2; a <= 8; ++a )
+            for ( int b = a; b <= a + 1 && b <= 8; ++b )
+            {
+                TileShape sh = { { a, b, c }, 0 };
+                if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, vals, order, sh ) >
+                     (size_t)scatter_lds( w ) )
+                    continue;
+                const double bricks = bricks_of( sh );
+                const double share = (double)( a * b ) / ( ( a + extra ) * ( b + extra ) );
+                const double score = share * ( bricks < 1024.0 ? bricks / 1024.0 : 1.0 );
+                if ( score <= best )
+                    continue;
+                best = score;
+                best_bricks = bricks;
+                found = true;
+                double cap = 1.25 * mean_ppc * a * b * c;
+                cap = cap < 1024 ? 1024 : ( cap > 8192 ? 8192 : cap );
+                sh.cap = ( (int)cap + 63 ) / 64 * 64;
+                out = sh;
+            }
+    }
     return found;
 }
 
@@ -814,7 +788,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
 // describe the mesh's own cells or the order has no tiled kernels (only
 // orders 1 to 3 do).
 bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
-                 const int* slot_ng, int nslot, int rec_len,
+                 const int* slot_ng, int nslot, int vals,
                  const cabana_amd_binning* bins, const GFieldDev& g0,
                  TileArgs& t, size_t& lds )
 {
@@ -828,7 +802,7 @@ bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
     const double ncell = (double)m.num_cell[0] * m.num_cell[1] * m.num_cell[2];
     const double mean_ppc = ncell > 0 ? (double)( bins->end - bins->begin ) / ncell : 0.0;
     TileShape sh;
-    if ( !choose_shape( kind, fp64, slot_ng, nslot, rec_len, order, mean_ppc, sh ) )
+    if ( !choose_shape( kind, fp64, slot_ng, nslot, vals, order, m.num_cell, mean_ppc, sh ) )
         return false;
     const int extra = ( order == 1 ) ? 1 : 3;
     std::memset( &t, 0, sizeof( t ) );
@@ -841,15 +815,8 @@ bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
         t.win[d] = sh.T[d] + extra;
     }
     t.max_runs = sh.T[0] * sh.T[1];
-    // The scatter keeps a run table in one wave (<= 64 runs) and base-cell
-    // coordinates in 4-bit task fields.
-    if ( kind == TILE_SCATTER &&
-         ( t.max_runs > 64 || sh.T[0] > 14 || sh.T[1] > 14 || sh.T[2] > 14 ) )
-        return false;
     t.max_win_nodes = t.win[0] * t.win[1] * t.win[2];
-    t.max_base_cells = base_cells( sh.T, order );
     t.cap = sh.cap;
-    t.max_tasks = sh.max_tasks;
     t.bin_begin = bins->begin;
     // Window walk order: largest grid stride first.
     int perm[3] = { 0, 1, 2 };
@@ -863,7 +830,7 @@ bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
             }
     for ( int d = 0; d < 3; ++d )
         t.flush_perm[d] = perm[d];
-    lds = tile_lds_bytes( kind, fp64, slot_ng, nslot, rec_len, order, sh );
+    lds = tile_lds_bytes( kind, fp64, slot_ng, nslot, vals, order, sh );
     return true;
 }
 
@@ -1027,16 +994,19 @@ cabana_amd_status scatter_pass( cabana_amd_context* ctx, int order, bool fp64,
     a.contig = pf_contig( a.points ) && pf_contig( a.xbar );
     for ( int i = 0; i < a.nterms; ++i )
         a.contig = a.contig && pf_contig( a.t[i].pin );
-    // Record header of the cell-tiled scatter: the x weights and gradients
-    // with the y and z offsets for FP32 records, the three offsets for FP64.
-    int rec_len = fp64 ? 3 : 2 * ( order + 1 ) + 2;
+    // Values of a record's slot: one for value-type terms, three for
+    // gradient-type ones (ScalarValue and VectorValue share theirs).
+    int vals = 0;
     for ( int i = 0; i < a.nterms; ++i )
-        rec_len += form_pcomp( forms[i] );
+        if ( forms[i] != FORM_SV && forms[i] != FORM_VV )
+            vals += 3;
+        else if ( i == 0 )
+            vals += 1;
     TileArgs t;
     size_t lds = 0;
     const bool tiled =
         !a.has_xbar && bins_usable( bins, n ) &&
-        make_tiles( TILE_SCATTER, a.mesh, order, fp64, ng, nslot, rec_len, bins,
+        make_tiles( TILE_SCATTER, a.mesh, order, fp64, ng, nslot, vals, bins,
                     a.t[0].grid, t, lds );
     if ( !tiled )
     {

@@ -49,6 +49,8 @@ struct PFieldDev
         const uint32_t p = (uint32_t)p64;
         return ( p >> shift ) * stride + ( p & mask );
     }
+    // base( p ) of a field with vector_length 1.
+    __device__ __forceinline__ uint32_t row( int64_t p ) const { return (uint32_t)p * stride; }
     template <class T>
     __device__ __forceinline__ T* ptr( uint32_t b, int c ) const
     {
@@ -141,13 +143,13 @@ __device__ __forceinline__ void vec_copy_out( const T* src, T* dst )
 template <class T, int N, bool CONTIG>
 __device__ __forceinline__ void PFieldDev::load( int64_t p, T* v ) const
 {
-    const uint32_t b = base( p );
     if constexpr ( CONTIG )
     {
-        detail::vec_copy_in<T, N>( ptr<const T>( b, 0 ), v );
+        detail::vec_copy_in<T, N>( ptr<const T>( row( p ), 0 ), v );
     }
     else
     {
+        const uint32_t b = base( p );
 #pragma unroll
         for ( int c = 0; c < N; ++c )
             v[c] = *ptr<const T>( b, c );
@@ -157,13 +159,13 @@ __device__ __forceinline__ void PFieldDev::load( int64_t p, T* v ) const
 template <class T, int N, bool CONTIG>
 __device__ __forceinline__ void PFieldDev::store( int64_t p, const T* v ) const
 {
-    const uint32_t b = base( p );
     if constexpr ( CONTIG )
     {
-        detail::vec_copy_out<T, N>( v, ptr<T>( b, 0 ) );
+        detail::vec_copy_out<T, N>( v, ptr<T>( row( p ), 0 ) );
     }
     else
     {
+        const uint32_t b = base( p );
 #pragma unroll
         for ( int c = 0; c < N; ++c )
             *ptr<T>( b, c ) = v[c];
@@ -349,9 +351,7 @@ struct TileArgs
     int32_t flush_perm[3];       // grid dims from largest to smallest stride
     int32_t max_runs;            // tile[0] * tile[1]
     int32_t max_win_nodes;       // win[0] * win[1] * win[2]
-    int32_t max_base_cells;      // stencil-base cells of a brick
     int32_t cap;                 // particles per part
-    int32_t max_tasks;           // scatter: task-table capacity
     int32_t grid;                // workgroups launched (a multiple of 8)
     int64_t bin_begin;           // particle index of cell offset 0
     // Particle at each binned position q (perm[q - bin_begin]) when the
@@ -364,23 +364,35 @@ struct TileArgs
     }
 };
 
-// LDS record of one particle in the cell-sorted scatter: 3 fractional
-// offsets then the premultiplied attributes, padded to 16 bytes so a record
-// is read with 128-bit LDS loads.  Records are read through a sorted index,
-// so no stride is free of bank conflicts and none is padded for it.
-__host__ __device__ constexpr int record_stride( int len, int elem_bytes )
+// Cell-tiled scatter (ca_scatter.hip).  A pass is of one of two kinds, by the
+// values in a slot of its records (scatter_row): four with value-type terms
+// only, six with gradient-type ones.
+constexpr int SCATTER_BLOCK = 256;
+constexpr int scatter_row( int vals ) { return ( 2 + vals + 1 ) / 2 * 2; }
+// Waves per SIMD the registers of a pass leave room for without spilling
+// (a spill of a few registers at one wave more measured 1.2 to 2 times
+// slower), and the LDS that lets as many workgroups run on a CU.
+constexpr int scatter_waves( bool fp64, int row )
 {
-    return ( len * elem_bytes + 15 ) / 16 * 16 / elem_bytes;
+    return fp64 ? ( row == 4 ? 3 : 2 ) : ( row == 4 ? 4 : 3 );
 }
-// Threads of a scatter workgroup (FP32 / FP64 records) and the particles
-// each thread holds per part; their product is the largest part.
-constexpr int scatter_block( bool fp64 ) { return 256; }
-constexpr int SCATTER_SLOTS = 2; // tested value; 3 failed the unbinned tests
-// Longest run of one base cell's records that one scatter task takes
-// (8 measured faster than 16 or 32 at 16 particles per cell: tasks of more
-// even length leave fewer lanes idle).
-constexpr int SCATTER_TASK_MAX = 8; // tested value; 12 failed the dense-cell tests
-constexpr int scatter_cap_max( bool fp64 ) { return scatter_block( fp64 ) * SCATTER_SLOTS; }
+constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
+// Particles of a wave's batch of 64 whose records are in LDS at a time.
+// Larger records leave the window too little room with 64 (and cost a wave per
+// SIMD); 16 break more groups apart: at 128^3 x 16 FP32 the MPM P2G takes
+// 1.51 ms with 32 and 1.67 ms with 16, and mass and momentum of 8.4 M clustered
+// particles, whose windows are larger, 0.50 ms with 32 and 0.46 ms with 16.
+constexpr int scatter_sub( int row ) { return row == 4 ? 16 : 32; }
+// Cells of a scatter brick along k, a compile-time stride of the LDS window
+// (linear splines: groups of three cells).
+constexpr int scatter_cells_k( int order ) { return order == 1 ? 9 : 8; }
+// A scatter record: 16 weights and four slot rows of `row` values, with a
+// stride that puts the 16-byte pieces eight lanes write at a time into
+// different LDS banks.
+constexpr int scatter_record( bool fp64, int row )
+{
+    return 16 + 4 * row + ( fp64 ? 2 : ( row == 4 ? 4 : 0 ) );
+}
 
 // Launch-time error/timing context owned by the C-ABI layer.
 class Launcher

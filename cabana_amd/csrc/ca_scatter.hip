@@ -1,0 +1,853 @@
+// Cell-tiled scatter of cell-sorted particles on the matrix cores, one spline
+// order per translation unit (CA_ORDER set on the compile line): P2G forward
+// and the grid part of the G2P adjoint.
+//
+// Every stencil of a particle of one mesh cell lies in the cell's 4^3 node
+// window (linear splines: the window of three cells along k).  With the 1-D
+// weights w and gradients g along the window padded by zeros, a node value is
+//   G[(i,j),(k,d)] = sum_p  (wx_i wy_j) (wz_k P1_d + gz_k P4_d)
+//                         + (gx_i wy_j) (wz_k P2_d) + (wx_i gy_j) (wz_k P3_d)
+// which is a matrix product over the particles with 16 rows (i, j) and 16
+// columns (k, d): v_mfma_*_16x16x4 takes four particles at a time, one product
+// for value-type dofs and three for gradient-type ones.  Particles are taken
+// in the order of the binning, so nothing is sorted in the kernel: a wave
+// walks its share of the part, 64 particles a batch (one per lane: positions,
+// weights and attributes, written to the wave's records in LDS), then the
+// batch's runs of equal cell, four particles a step.
+#include "ca_tiles.hpp"
+
+namespace cabana_amd
+{
+namespace
+{
+
+// Columns of the matrix product.  A tile is one 16 x 16 accumulator: columns
+// (k, slot) of four window nodes and four slots, each slot a grid dof.  The
+// ScalarValue and VectorValue terms of a fused P2G share a tile (slot 0 and
+// slots 1 to 3); every other form has its dofs in slots 0 to 2.
+template <bool SHARED, int... FORMS>
+struct Tiles
+{
+    using FL = FormList<FORMS...>;
+    static constexpr bool PAIR = !SHARED && FL::N >= 2;
+    static constexpr int NT = SHARED ? 1 : ( FL::N == 3 ? 2 : 1 );
+    static constexpr int first_term( int tile ) { return tile == 0 ? 0 : 2; }
+    static constexpr int last_term( int tile )
+    {
+        return SHARED ? FL::N - 1 : ( tile == 0 ? ( PAIR ? 1 : 0 ) : 2 );
+    }
+    static constexpr bool value_form( int f ) { return f == FORM_SV || f == FORM_VV; }
+    // Slots of a tile that hold a dof.
+    static constexpr int nd( int tile )
+    {
+        return ( PAIR && tile == 0 ) ? 4 : ng_of( FL::v[last_term( tile )] );
+    }
+    // The tile has value-type (P1) and gradient-type (P2, P3, P4) columns.
+    static constexpr bool has_v( int tile )
+    {
+        bool r = false;
+        for ( int t = first_term( tile ); t <= last_term( tile ); ++t )
+            r = r || value_form( FL::v[t] );
+        return r;
+    }
+    static constexpr bool has_g( int tile )
+    {
+        bool r = false;
+        for ( int t = first_term( tile ); t <= last_term( tile ); ++t )
+            r = r || !value_form( FL::v[t] );
+        return r;
+    }
+    // Offset of a tile's values in a record's slot row, after its weight and
+    // gradient.
+    static constexpr int val( int tile )
+    {
+        int o = 2;
+        for ( int i = 0; i < tile; ++i )
+            o += ( has_v( i ) ? 1 : 0 ) + ( has_g( i ) ? 3 : 0 );
+        return o;
+    }
+    static constexpr int row_len() { return val( NT ); }
+    static constexpr int row() { return ( row_len() + 1 ) / 2 * 2; }
+    static constexpr int win_dofs()
+    {
+        int n = 0;
+        for ( int i = 0; i < NT; ++i )
+            n += nd( i );
+        return n;
+    }
+};
+
+// Record of a particle: weight and gradient along QUAD and along k of the four
+// window nodes, then the four slot rows (weight and gradient along SLOT of the
+// node with the slot's number, then the slot's values) in 16-byte chunks,
+// [chunk][slot].  The record stride spreads the four records of a step over
+// the LDS banks.
+template <class Real, int ROW>
+struct Record
+{
+    static constexpr int CW = 16 / (int)sizeof( Real );
+    static constexpr int NC = ( ROW + CW - 1 ) / CW;
+    static constexpr int STRIDE = scatter_record( sizeof( Real ) == 8, ROW );
+    static constexpr int width( int c ) { return ROW - c * CW < CW ? ROW - c * CW : CW; }
+    static constexpr int at( int c, int slot ) { return 16 + 4 * CW * c + slot * width( c ); }
+    template <int N>
+    struct Vec
+    {
+        typedef Real type __attribute__( ( ext_vector_type( N ) ) );
+    };
+    static __device__ __forceinline__ void put_row( Real* rec, int slot, const Real* v )
+    {
+        static_for<NC>( [&]( auto C ) {
+            constexpr int c = C;
+            typename Vec<width( c )>::type x;
+#pragma unroll
+            for ( int e = 0; e < width( c ); ++e )
+                x[e] = v[c * CW + e];
+            *reinterpret_cast<typename Vec<width( c )>::type*>( rec + at( c, slot ) ) = x;
+        } );
+    }
+    static __device__ __forceinline__ void put_pair( Real* at, Real w, Real g )
+    {
+        *reinterpret_cast<typename Vec<2>::type*>( at ) = typename Vec<2>::type{ w, g };
+    }
+    static __device__ __forceinline__ void get_row( const Real* rec, int slot, Real* v )
+    {
+        static_for<NC>( [&]( auto C ) {
+            constexpr int c = C;
+            const auto x = *reinterpret_cast<const typename Vec<width( c )>::type*>( rec + at( c, slot ) );
+#pragma unroll
+            for ( int e = 0; e < width( c ); ++e )
+                v[c * CW + e] = x[e];
+        } );
+    }
+};
+
+// The slot values of form FORM: r[0] = P1 (value-type) or r = (P2, P3, P4).
+template <int FORM, class Real>
+__device__ __forceinline__ void slot_values( const Real* P, int d, Real* r )
+{
+    if constexpr ( FORM == FORM_SV || FORM == FORM_VV )
+        r[0] = P[d];
+    else if constexpr ( FORM == FORM_SG )
+    {
+        r[0] = d == 0 ? P[0] : Real( 0 );
+        r[1] = d == 1 ? P[0] : Real( 0 );
+        r[2] = d == 2 ? P[0] : Real( 0 );
+    }
+    else if constexpr ( FORM == FORM_VD )
+    {
+#pragma unroll
+        for ( int b = 0; b < 3; ++b )
+            r[b] = P[b];
+    }
+    else if constexpr ( FORM == FORM_TD )
+    {
+#pragma unroll
+        for ( int b = 0; b < 3; ++b )
+            r[b] = P[3 * d + b];
+    }
+    else
+    {
+#pragma unroll
+        for ( int b = 0; b < 3; ++b )
+            r[b] = P[3 * b + d];
+    }
+}
+
+// Matrix product of four particles.  Row rho of lane l's accumulator register
+// r is 4 (l / 16) + r in FP32 and l / 16 + 4 r in FP64.  Window node i sits in
+// lanes l / 16 = i and node j in register r = j either way: rho / 4 and rho % 4
+// are (i, j) in FP32 and (j, i) in FP64.  QUAD is the dimension along rho / 4
+// (one weight per quad of a row of 16 lanes), SLOT the one along rho % 4.
+template <class Real>
+struct Mfma;
+template <>
+struct Mfma<float>
+{
+    typedef float V4 __attribute__( ( ext_vector_type( 4 ) ) );
+    static constexpr int QUAD = 0, SLOT = 1;
+    static __device__ __forceinline__ V4 mac( float a, float b, V4 c )
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32( a, b, c, 0, 0, 0 );
+    }
+};
+template <>
+struct Mfma<double>
+{
+    typedef double V4 __attribute__( ( ext_vector_type( 4 ) ) );
+    static constexpr int QUAD = 1, SLOT = 0;
+    static __device__ __forceinline__ V4 mac( double a, double b, V4 c )
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64( a, b, c, 0, 0, 0 );
+    }
+};
+
+// DPP move: lane Q of every quad to its four lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp( float x )
+{
+    return __builtin_bit_cast( float, __builtin_amdgcn_update_dpp(
+        0, __builtin_bit_cast( int, x ), CTRL, 0xf, 0xf, true ) );
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp( double x )
+{
+    typedef int I2 __attribute__( ( ext_vector_type( 2 ) ) );
+    const I2 v = __builtin_bit_cast( I2, x );
+    I2 r;
+    r.x = __builtin_amdgcn_update_dpp( 0, v.x, CTRL, 0xf, 0xf, true );
+    r.y = __builtin_amdgcn_update_dpp( 0, v.y, CTRL, 0xf, 0xf, true );
+    return __builtin_bit_cast( double, r );
+}
+template <int Q, class Real>
+__device__ __forceinline__ Real quad_lane( Real x )
+{
+    return dpp<Q * 0x55>( x );
+}
+// Attributes of a pass: every term's components in order.
+template <int... FORMS>
+constexpr int attr_len()
+{
+    return ( np_of( FORMS ) + ... );
+}
+template <int... FORMS>
+constexpr int attr_of( int t )
+{
+    constexpr int f[] = { FORMS... };
+    int o = 0;
+    for ( int i = 0; i < t; ++i )
+        o += np_of( f[i] );
+    return o;
+}
+
+// Global-atomic scatter of one particle (particles whose stencil is outside
+// the brick's window, or whose attributes are not finite).  Rare, so its
+// loops stay rolled: unrolled, their registers would bound the kernel's.
+template <class Real, bool SHARED, int... FORMS>
+__device__ __forceinline__ void global_scatter_particle( const ScatterArgs& a, const double x[3],
+                                                         const Real* P )
+{
+    using FL = FormList<FORMS...>;
+    Spline3D<ORDER, Real, false> s;
+    eval_spline( a.mesh, x, s );
+#pragma unroll 1
+    for ( int n = 0; n < K * K * K; ++n )
+    {
+        const int i = n / ( K * K ), j = n / K % K, k = n % K;
+        Spline3D<0, Real, false> one;
+#pragma unroll
+        for ( int q = 0; q < K; ++q )
+        {
+            one.d[0].w[0] = q == 0 || i == q ? s.d[0].w[q] : one.d[0].w[0];
+            one.d[0].g[0] = q == 0 || i == q ? s.d[0].g[q] : one.d[0].g[0];
+            one.d[1].w[0] = q == 0 || j == q ? s.d[1].w[q] : one.d[1].w[0];
+            one.d[1].g[0] = q == 0 || j == q ? s.d[1].g[q] : one.d[1].g[0];
+            one.d[2].w[0] = q == 0 || k == q ? s.d[2].w[q] : one.d[2].w[0];
+            one.d[2].g[0] = q == 0 || k == q ? s.d[2].g[q] : one.d[2].g[0];
+        }
+        const auto nw = node_weights<0, Real, false, false>( one, 0, 0, 0 );
+        static_for<FL::N>( [&]( auto I ) {
+            constexpr int t = I;
+            constexpr int FORM = FL::v[t];
+            constexpr int NG = ng_of( FORM );
+            const GFieldDev& g = SHARED ? a.t[0].grid : a.t[t].grid;
+            Real G[NG];
+            form_scatter<FORM>( P + attr_of<FORMS...>( t ), nw, G );
+            Real* q = gptr<Real>( g, ( s.d[0].base + i ) * g.s[0] + ( s.d[1].base + j ) * g.s[1] +
+                                         ( s.d[2].base + k ) * g.s[2] );
+#pragma unroll
+            for ( int d = 0; d < NG; ++d )
+                atomic_add( q + d * g.s[3], G[d] );
+        } );
+    }
+}
+
+// The run table of a brick in two halves, so its global reads can be issued
+// early and committed later: lane r < nruns (<= 64) of wave 0 holds run r's
+// raw reads (nothing is computed from them until the commit, so issuing
+// them does not wait for them).
+struct RunLoad
+{
+    int64_t start;
+    int64_t last_offset;
+    int32_t last_count;
+};
+
+__device__ __forceinline__ void runs_issue( const TileArgs& ta, const MeshDev& m,
+                                            const TileGeom& g, RunLoad& rl )
+{
+    const int nj = g.c1[1] - g.c0[1];
+    const int nruns = ( g.c1[0] - g.c0[0] ) * nj;
+    const int r = threadIdx.x;
+    rl.start = 0;
+    rl.last_offset = 0;
+    rl.last_count = 0;
+    if ( r < nruns )
+    {
+        const int ci = g.c0[0] + r / nj, cj = g.c0[1] + r % nj;
+        const int64_t cfirst = ( (int64_t)ci * m.num_cell[1] + cj ) * m.num_cell[2] + g.c0[2];
+        const int64_t clast = cfirst + ( g.c1[2] - g.c0[2] ) - 1;
+        rl.start = ta.cell_offsets[cfirst];
+        rl.last_offset = ta.cell_offsets[clast];
+        rl.last_count = ta.cell_counts[clast];
+    }
+}
+
+// Wave 0 writes run_start and the inclusive prefix run_pre (visible after
+// the next barrier).
+__device__ __forceinline__ void runs_commit( const RunLoad& rl, const TileGeom& g,
+                                             int64_t* run_start, int* run_pre )
+{
+    if ( threadIdx.x >= 64 )
+        return;
+    const int nruns = ( g.c1[0] - g.c0[0] ) * ( g.c1[1] - g.c0[1] );
+    const int lane = threadIdx.x;
+    int v = (int)( rl.last_offset + rl.last_count - rl.start );
+#pragma unroll
+    for ( int o = 1; o < 64; o <<= 1 )
+    {
+        const int u = __shfl_up( v, o, 64 );
+        if ( lane >= o )
+            v += u;
+    }
+    if ( lane < nruns )
+    {
+        run_start[lane] = rl.start;
+        run_pre[lane + 1] = v;
+    }
+    if ( lane == 0 )
+        run_pre[0] = 0;
+}
+
+__device__ __forceinline__ float fabs_r( float x ) { return __builtin_fabsf( x ); }
+__device__ __forceinline__ double fabs_r( double x ) { return __builtin_fabs( x ); }
+
+// Particles of one batch between their loads and their use (the loads of the
+// next batch are in flight while this one is accumulated).
+template <class Real, int NP>
+struct Batch
+{
+    double x[3];
+    Real attr[NP];
+};
+
+// Issues the reads of the particle at flattened part position v, run r being a
+// run at or before its own.  Every lane reads a particle (past the end, the
+// last one), so that nothing of the batch before stays live.
+template <class Real, bool CONTIG, int... FORMS>
+__device__ __forceinline__ void batch_issue( const ScatterArgs& a, const TileArgs& ta,
+                                             const int64_t* run_start, const int* run_pre,
+                                             int v, int v1, int& r,
+                                             Batch<Real, attr_len<FORMS...>()>& b )
+{
+    v = min( v, v1 - 1 );
+    while ( run_pre[r + 1] <= v )
+        ++r;
+    const int64_t p = ta.particle( ta.bin_begin + run_start[r] + ( v - run_pre[r] ) );
+    load_position<CONTIG>( a.points, p, b.x );
+    using FL = FormList<FORMS...>;
+    static_for<FL::N>( [&]( auto I ) {
+        constexpr int t = I;
+        a.t[t].pin.template load<Real, np_of( FL::v[t] ), CONTIG>( p,
+                                                                   b.attr + attr_of<FORMS...>( t ) );
+    } );
+}
+
+// Weights along a group's four window nodes, zero outside the stencil, which
+// starts off nodes into the window.
+template <class Real>
+__device__ __forceinline__ void window_weights( const Real* s, int off, Real* w )
+{
+#pragma unroll
+    for ( int n = 0; n < 4; ++n )
+    {
+        Real v = n < K ? s[n < K ? n : 0] : Real( 0 );
+        if constexpr ( ORDER <= 2 )
+        {
+            const Real v1 = ( n >= 1 && n - 1 < K ) ? s[n >= 1 ? n - 1 : 0] : Real( 0 );
+            v = off == 1 ? v1 : v;
+        }
+        if constexpr ( ORDER == 1 )
+        {
+            const Real v2 = n >= 2 ? s[n >= 2 ? n - 2 : 0] : Real( 0 );
+            v = off == 2 ? v2 : v;
+        }
+        w[n] = v;
+    }
+}
+
+// Window nodes along k (a compile-time stride of the LDS window).
+constexpr int WK = scatter_cells_k( ORDER ) + ( ORDER == 1 ? 1 : 3 );
+
+// A step's operands as read from the records.
+template <class Real, int ROW>
+struct Step
+{
+    Real xz;
+    Real y[ROW];
+};
+
+template <class Real, bool CONTIG, bool SHARED, int... FORMS>
+__global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 8, Tiles<SHARED, FORMS...>::row() ) ) ) void scatter_cells_kernel(
+    ScatterArgs a, TileArgs ta )
+{
+    using FL = FormList<FORMS...>;
+    using TL = Tiles<SHARED, FORMS...>;
+    using MF = Mfma<Real>;
+    using V4 = typename MF::V4;
+    constexpr int NT = TL::NT;
+    constexpr int ROW = TL::row();
+    using RC = Record<Real, ROW>;
+    constexpr int RS = RC::STRIDE;
+    constexpr int NP = attr_len<FORMS...>();
+    constexpr int NWAVE = SCATTER_BLOCK / 64;
+    constexpr int SUB = scatter_sub( ROW );
+    constexpr bool F32 = sizeof( Real ) == 4;
+    // Window nodes along k sit in column (node index mod 4), so that the
+    // window slides to the next cell without moving the accumulators.  (The
+    // windows of the linear spline are three cells apart and do not slide.)
+    constexpr bool SLIDE = ORDER != 1;
+    extern __shared__ __align__( 16 ) unsigned char smem[];
+
+    // LDS: the FP64 node window (one block per tile, [node][dof]), the waves'
+    // records, the run table.
+    const int W[3] = { ta.win[0], ta.win[1], WK };
+    const int wnodes = W[0] * W[1] * W[2];
+    double* win = reinterpret_cast<double*>( smem );
+    size_t off = align16( sizeof( double ) * (size_t)TL::win_dofs() * ta.max_win_nodes );
+    const int lane = (int)threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane( (int)threadIdx.x >> 6 );
+    Real* rec = reinterpret_cast<Real*>( smem + off ) + wave * ( RS * ( SUB + 3 ) );
+    off = align16( off + sizeof( Real ) * (size_t)NWAVE * RS * ( SUB + 3 ) );
+    int64_t* run_start = reinterpret_cast<int64_t*>( smem + off );
+    off = align16( off + sizeof( int64_t ) * ta.max_runs );
+    int* run_pre = reinterpret_cast<int*>( smem + off );
+
+    // The lane's place in the products: particle of a step, window row or
+    // column, dof slot; and in the accumulators.
+    const int pslot = lane >> 4, l16 = lane & 15, kcol = l16 >> 2, slot = lane & 3;
+
+    for ( int e = threadIdx.x; e < TL::win_dofs() * wnodes; e += SCATTER_BLOCK )
+        win[e] = 0.0;
+    // Records past a group are read (and count zero): they hold finite values.
+    for ( int e = lane; e < RS * ( SUB + 3 ); e += 64 )
+        rec[e] = Real( 0 );
+
+    const Real vmax = Real( sizeof( Real ) == 8 ? 1e300 : 1e30 ) /
+                      ( Real( 1 ) + (Real)a.mesh.rdx[0] + (Real)a.mesh.rdx[1] + (Real)a.mesh.rdx[2] );
+
+    const PartLoop pl( ta );
+    for ( int loc = pl.first; pl.more( loc ); loc += pl.stride )
+    {
+        const int w = pl.part( loc );
+        if ( w < 0 )
+            continue;
+        TileGeom tg;
+        part_geometry( ta, a.mesh, w, tg );
+        if ( threadIdx.x < 64 )
+        {
+            RunLoad rl;
+            runs_issue( ta, a.mesh, tg, rl );
+            runs_commit( rl, tg, run_start, run_pre );
+        }
+        __syncthreads();
+        // Window origin, and the stencil bases (from it) whose nodes lie in the
+        // window and in the grid.
+        int wlo[3], rmin[3], rcount[3];
+#pragma unroll
+        for ( int d = 0; d < 3; ++d )
+        {
+            wlo[d] = tg.c0[d] + a.mesh.halo + BASE_SHIFT;
+            rmin[d] = max( 0, -wlo[d] );
+            rcount[d] = max( 0, min( W[d], a.mesh.num_node[d] - wlo[d] ) - K + 1 - rmin[d] );
+        }
+        const int nruns = ( tg.c1[0] - tg.c0[0] ) * ( tg.c1[1] - tg.c0[1] );
+        const int pbeg = tg.part * ta.cap;
+        const int pend = min( run_pre[nruns], pbeg + ta.cap );
+        // The wave's share: a contiguous range of whole batches.
+        const int per = ( ( pend - pbeg + NWAVE * 64 - 1 ) / ( NWAVE * 64 ) ) * 64;
+        const int v0 = __builtin_amdgcn_readfirstlane( pbeg + wave * per );
+        const int v1 = __builtin_amdgcn_readfirstlane( min( pend, v0 + per ) );
+
+        // The open window: key of the group in the accumulators, -1 none.
+        int open = -1;
+        double acc[NT][4];
+#pragma unroll
+        for ( int t = 0; t < NT; ++t )
+#pragma unroll
+            for ( int r = 0; r < 4; ++r )
+                acc[t][r] = 0.0;
+        // Adds the accumulators to the LDS window (all columns, or the window's
+        // first node along k) and clears them.
+        auto retire = [&]( int key, bool all ) {
+            const int dk = SLIDE ? ( kcol - key ) & 3 : kcol;
+            const int node = ( ( ( key >> 16 ) + pslot ) * W[1] + ( ( key >> 8 ) & 255 ) ) * WK +
+                             ( key & 255 ) + dk;
+            const bool on = ( all || dk == 0 ) && ( ORDER > 1 || pslot < 2 );
+            int wo = 0;
+            static_for<NT>( [&]( auto T ) {
+                constexpr int t = T;
+                constexpr int ND = TL::nd( t );
+                if ( on && ( ND == 4 || slot < ND ) )
+                {
+                    double* q = win + ( wo + node * ND + slot );
+#pragma unroll
+                    for ( int r = 0; r < ( ORDER > 1 ? 4 : 2 ); ++r )
+                        atomicAdd( q + r * WK * ND, acc[t][r] );
+                }
+                wo += ta.max_win_nodes * ND;
+            } );
+            if ( on )
+            {
+#pragma unroll
+                for ( int t = 0; t < NT; ++t )
+#pragma unroll
+                    for ( int r = 0; r < 4; ++r )
+                        acc[t][r] = 0.0;
+            }
+        };
+
+        Batch<Real, NP> bt;
+        int run = 0;
+        if ( v0 < v1 )
+        {
+            run = find_run( run_pre, nruns, v0 );
+            batch_issue<Real, CONTIG, FORMS...>( a, ta, run_start, run_pre, v0 + lane, v1, run, bt );
+        }
+        for ( int vb = v0; vb < v1; vb += 64 )
+        {
+            // Particle phase: stencil base, weights, premultiplied attributes.
+            // key: window origin of the particle's group, -1 for none.
+            int key = -1;
+            Real wt[3][4], gt[3][4], P[NP];
+            if ( vb + lane < v1 )
+            {
+                int org[3];
+                bool fits = true;
+#pragma unroll
+                for ( int d = 0; d < 3; ++d )
+                {
+                    // spline_frac without its early returns.
+                    const double x0 = logical_coord<ORDER>( bt.x[d], a.mesh.low[d], a.mesh.rdx[d] );
+                    const int i0 = (int)x0;
+                    const Real fr = (Real)( x0 - (double)i0 );
+                    const int rel = i0 - ORDER / 2 - wlo[d];
+                    fits = fits && x0 >= 0.0 && x0 < 2147483648.0 &&
+                           (unsigned)( rel - rmin[d] ) < (unsigned)rcount[d];
+                    int l = rel;
+                    if constexpr ( ORDER == 2 )
+                        l = min( max( rel - ( fr < Real( 0.5 ) ? 1 : 0 ), 0 ), W[d] - 4 );
+                    if constexpr ( ORDER == 1 )
+                        l = d == 2 ? (int)( (unsigned)rel / 3u * 3u ) : rel;
+                    org[d] = l;
+                    Spline1D<ORDER, Real> sd;
+                    spline_weights<ORDER, Real, false>( fr, (Real)a.mesh.rdx[d], sd );
+                    window_weights( sd.w, rel - l, wt[d] );
+                    window_weights( sd.g, rel - l, gt[d] );
+                }
+                Real big = Real( 0 );
+                static_for<FL::N>( [&]( auto I ) {
+                    constexpr int t = I;
+                    constexpr int o = attr_of<FORMS...>( t );
+                    const Real m = (Real)a.t[t].mult;
+#pragma unroll
+                    for ( int c = 0; c < np_of( FL::v[t] ); ++c )
+                    {
+                        P[o + c] = bt.attr[o + c] * m;
+                        big += fabs_r( P[o + c] );
+                    }
+                } );
+                // A value that is not finite, or overflows against a weight
+                // gradient, must not meet the zero weights of window nodes
+                // outside its stencil.
+                if ( fits && big <= vmax )
+                    key = ( org[0] << 16 ) | ( org[1] << 8 ) | org[2];
+                else
+                {
+                    int base[3];
+                    if ( stencil_base<ORDER>( a.mesh, bt.x, base ) )
+                        global_scatter_particle<Real, SHARED, FORMS...>( a, bt.x, P );
+                    else
+                        atomicAdd( a.skipped, 1ull );
+                }
+            }
+            const int nb = min( 64, v1 - vb );
+            const int before = __shfl_up( key, 1, 64 );
+            const uint64_t starts = __ballot( lane == 0 || key != before );
+
+            static_for<64 / SUB>( [&]( auto IS ) {
+                constexpr int s0 = IS * SUB;
+                if ( s0 >= nb )
+                    return;
+                if ( ( lane & ~( SUB - 1 ) ) == s0 && key >= 0 )
+                {
+                    Real* rp = rec + ( lane - s0 ) * RS;
+#pragma unroll
+                    for ( int n = 0; n < 4; ++n )
+                    {
+                        RC::put_pair( rp + 4 * n, wt[MF::QUAD][n], gt[MF::QUAD][n] );
+                        RC::put_pair( rp + 4 * ( SLIDE ? ( key + n ) & 3 : n ) + 2, wt[2][n],
+                                      gt[2][n] );
+                    }
+                    static_for<4>( [&]( auto S ) {
+                        constexpr int sl = S;
+                        Real v[ROW];
+                        v[0] = wt[MF::SLOT][sl];
+                        v[1] = gt[MF::SLOT][sl];
+#pragma unroll
+                        for ( int c = 2; c < ROW; ++c )
+                            v[c] = Real( 0 );
+                        if constexpr ( TL::PAIR )
+                        {
+                            v[2] = P[sl];
+                            if constexpr ( NT == 2 && sl < 3 )
+                                slot_values<FL::v[FL::N - 1]>( P + 4, sl, v + TL::val( 1 ) );
+                        }
+                        else
+                            static_for<FL::N>( [&]( auto I ) {
+                                constexpr int t = I;
+                                constexpr int F = FL::v[t];
+                                if constexpr ( sl < ng_of( F ) )
+                                    slot_values<F>( P + attr_of<FORMS...>( t ), sl,
+                                                    v + 2 + ( SHARED && t == 1 ? 1 : 0 ) );
+                            } );
+                        RC::put_row( rp, sl, v );
+                    } );
+                }
+                __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+                __builtin_amdgcn_wave_barrier();
+                // The next batch's reads complete while the last records
+                // accumulate (issued here, where this batch's registers are
+                // free).
+                if constexpr ( s0 + SUB == 64 )
+                    batch_issue<Real, CONTIG, FORMS...>( a, ta, run_start, run_pre, vb + 64 + lane,
+                                                         v1, run, bt );
+                const int s1 = min( s0 + SUB, nb );
+                int s = s0;
+                while ( s < s1 )
+                {
+                    const uint64_t rest = s < 63 ? starts >> ( s + 1 ) : 0;
+                    const int e = rest ? min( s1, s + 1 + __builtin_ctzll( rest ) ) : s1;
+                    const int gk = __builtin_amdgcn_readlane( key, s );
+                    if ( gk < 0 )
+                    {
+                        s = e;
+                        continue;
+                    }
+                    // The group's window: the open one, or the next along k
+                    // (one node leaves the accumulators), or a new one.
+                    if ( gk != open )
+                    {
+                        if ( open >= 0 )
+                            retire( open, !( SLIDE && gk == open + 1 ) );
+                        open = gk;
+                    }
+                    int n = e - s;
+                    const Real* rp = rec + ( s - s0 + pslot ) * RS;
+                    s = e;
+                    while ( n > 0 )
+                    {
+                        // FP32 products are summed over 16 particles at most,
+                        // a gradient-type tile's three kinds apart, and the
+                        // sums added in FP64 (one FP32 sum of all three was
+                        // less accurate than the kernel before this one; its
+                        // products also wait for each other).  Each count of
+                        // steps is code of its own, without branches, so that
+                        // its operand reads are issued together: 1.87 -> 1.62
+                        // ms against a loop that read a step ahead.
+                        auto chunk = [&]( auto STEPS ) {
+                            constexpr int NS = STEPS;
+                            V4 D[NT][3];
+                            Step<Real, ROW> st[NS];
+                            static_for<NS>( [&]( auto C ) {
+                                constexpr int c = C;
+                                st[c].xz = rp[4 * c * RS + l16];
+                                RC::get_row( rp + 4 * c * RS, slot, st[c].y );
+                            } );
+                            __builtin_amdgcn_sched_barrier( 0 );
+                            static_for<NS>( [&]( auto C ) {
+                                constexpr int c = C;
+                                // Particles past the group count zero.
+                                Real xz = st[c].xz;
+                                if ( c == NS - 1 )
+                                    xz = pslot < n - 4 * c ? xz : Real( 0 );
+                                const Real wq = quad_lane<0>( xz ), gq = quad_lane<1>( xz );
+                                const Real wz = quad_lane<2>( xz ), gz = quad_lane<3>( xz );
+                                const Real A1 = wq * st[c].y[0], AQ = gq * st[c].y[0],
+                                           AS = wq * st[c].y[1];
+                                Real B[NT][3];
+                                static_for<NT>( [&]( auto T ) {
+                                    constexpr int t = T;
+                                    const Real* v = st[c].y + TL::val( t );
+                                    if constexpr ( !TL::has_g( t ) )
+                                        B[t][0] = wz * v[0];
+                                    else
+                                    {
+                                        const Real* h = v + ( TL::has_v( t ) ? 1 : 0 );
+                                        B[t][0] = gz * h[2];
+                                        if constexpr ( TL::has_v( t ) )
+                                            B[t][0] += wz * v[0];
+                                        B[t][1] = wz * h[MF::QUAD];
+                                        B[t][2] = wz * h[MF::SLOT];
+                                    }
+                                } );
+                                static_for<NT>( [&]( auto T ) {
+                                    constexpr int t = T;
+                                    constexpr int m1 = 1, m2 = F32 ? 2 : 1;
+                                    if constexpr ( c == 0 )
+                                    {
+                                        D[t][0] = D[t][1] = D[t][2] = V4{ 0, 0, 0, 0 };
+                                        if constexpr ( !F32 )
+                                            D[t][0] =
+                                                V4{ acc[t][0], acc[t][1], acc[t][2], acc[t][3] };
+                                    }
+                                    D[t][0] = MF::mac( A1, B[t][0], D[t][0] );
+                                    if constexpr ( TL::has_g( t ) )
+                                    {
+                                        D[t][m1] = MF::mac( AQ, B[t][1], D[t][m1] );
+                                        D[t][m2] = MF::mac( AS, B[t][2], D[t][m2] );
+                                    }
+                                } );
+                            } );
+                            static_for<NT>( [&]( auto T ) {
+                                constexpr int t = T;
+#pragma unroll
+                                for ( int r = 0; r < 4; ++r )
+                                    if constexpr ( !F32 )
+                                        acc[t][r] = TL::has_g( t ) ? D[t][0][r] + D[t][1][r]
+                                                                   : D[t][0][r];
+                                    else if constexpr ( TL::has_g( t ) )
+                                        acc[t][r] +=
+                                            (double)( ( D[t][0][r] + D[t][1][r] ) + D[t][2][r] );
+                                    else
+                                        acc[t][r] += (double)D[t][0][r];
+                            } );
+                        };
+                        if ( n > 12 )
+                            chunk( std::integral_constant<int, 4>{} );
+                        else if ( n > 8 )
+                            chunk( std::integral_constant<int, 3>{} );
+                        else if ( n > 4 )
+                            chunk( std::integral_constant<int, 2>{} );
+                        else
+                            chunk( std::integral_constant<int, 1>{} );
+                        n -= 16;
+                        rp += 16 * RS;
+                    }
+                }
+                // The records are rewritten by the next sub-batch.
+                __builtin_amdgcn_fence( __ATOMIC_ACQ_REL, "wavefront" );
+                __builtin_amdgcn_wave_barrier();
+            } );
+        }
+        if ( open >= 0 )
+            retire( open, true );
+        __syncthreads();
+
+        // Flush the window, one thread per node (the grid's unit-stride
+        // dimension fastest across threads): the node's dofs are read and
+        // zeroed for the next part, and every non-zero value is added to its
+        // grid with one global atomic.
+        const float rW[3] = { 1.0f / (float)W[0], 1.0f / (float)W[1], 1.0f / (float)W[2] };
+        for ( int f = threadIdx.x; f < wnodes; f += SCATTER_BLOCK )
+        {
+            int q[3], d0;
+            window_coords<1>( ta, f, W, rW, q, d0 );
+            const int node = ( q[0] * W[1] + q[1] ) * W[2] + q[2];
+            const int gi = wlo[0] + q[0], gj = wlo[1] + q[1], gk = wlo[2] + q[2];
+            const bool in = gi >= 0 && gj >= 0 && gk >= 0 && gi < a.mesh.num_node[0] &&
+                            gj < a.mesh.num_node[1] && gk < a.mesh.num_node[2];
+            int wo = 0;
+            static_for<NT>( [&]( auto T ) {
+                constexpr int t = T;
+                constexpr int ND = TL::nd( t );
+                double* src = win + ( wo + node * ND );
+                wo += ta.max_win_nodes * ND;
+                double v[ND];
+#pragma unroll
+                for ( int d = 0; d < ND; ++d )
+                {
+                    v[d] = src[d];
+                    src[d] = 0.0;
+                }
+                if ( in )
+                    static_for<ND>( [&]( auto D ) {
+                        constexpr int d = D;
+                        constexpr bool vec = TL::PAIR && t == 0 && d > 0;
+                        const GFieldDev& g = a.t[vec ? 1 : TL::first_term( t )].grid;
+                        const Real x = (Real)v[d];
+                        if ( x != Real( 0 ) )
+                            atomic_add( gptr<Real>( g, gi * g.s[0] + gj * g.s[1] + gk * g.s[2] +
+                                                           ( vec ? d - 1 : d ) * g.s[3] ),
+                                        x );
+                    } );
+            } );
+        }
+        // The next part reuses the window and the run table.
+        __syncthreads();
+    }
+}
+
+template <class Real, bool CONTIG>
+hipError_t scatter_cells_launch( int plan, const ScatterArgs& a, const TileArgs& t, size_t lds,
+                                 hipStream_t s )
+{
+    if ( plan == PLAN_SINGLE )
+    {
+        switch ( a.t[0].form )
+        {
+#define CA_CASE( F )                                                           \
+    case F:                                                                    \
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, F>, a, t, lds, s, SCATTER_BLOCK );
+            CA_CASE( FORM_SV )
+            CA_CASE( FORM_VV )
+            CA_CASE( FORM_SG )
+            CA_CASE( FORM_VD )
+            CA_CASE( FORM_TD )
+            CA_CASE( FORM_TDT )
+#undef CA_CASE
+        default:
+            return hipErrorInvalidValue;
+        }
+    }
+    if ( plan == PLAN_MPM_P2G )
+        return launch_tile_kernel(
+            scatter_cells_kernel<Real, CONTIG, false, FORM_SV, FORM_VV, FORM_TD>, a, t, lds, s,
+            SCATTER_BLOCK );
+    if ( plan == PLAN_MASS_MOMENTUM )
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, FORM_SV, FORM_VV>,
+                                   a, t, lds, s, SCATTER_BLOCK );
+    if ( plan == PLAN_MPM_G2P )
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, true, FORM_VV, FORM_TDT>,
+                                   a, t, lds, s, SCATTER_BLOCK );
+    return hipErrorInvalidValue;
+}
+
+template <class Real>
+hipError_t scatter_cells_typed( Launcher& L, int plan, const ScatterArgs& a,
+                                const TileArgs& t, size_t lds, hipStream_t s )
+{
+    const char* name = plan == PLAN_MPM_P2G         ? "p2g_mpm_cells"
+                       : plan == PLAN_MPM_G2P       ? "g2p_adjoint_mpm_cells"
+                       : plan == PLAN_MASS_MOMENTUM ? "p2g_mass_momentum_cells"
+                                                    : "scatter_cells";
+    L.before( name, s );
+    const hipError_t e = a.contig ? scatter_cells_launch<Real, true>( plan, a, t, lds, s )
+                                  : scatter_cells_launch<Real, false>( plan, a, t, lds, s );
+    L.after( name, s );
+    return e;
+}
+
+} // namespace
+
+hipError_t CA_CAT( launch_scatter_cells_, CA_SUFFIX )( Launcher& L, bool fp64,
+                                                      int plan,
+                                                      const ScatterArgs& a,
+                                                      const TileArgs& t,
+                                                      size_t lds, hipStream_t s )
+{
+    return fp64 ? scatter_cells_typed<double>( L, plan, a, t, lds, s )
+                : scatter_cells_typed<float>( L, plan, a, t, lds, s );
+}
+
+} // namespace cabana_amd

@@ -1,0 +1,96 @@
+"""The cell-tiled P2G scatter where its groups of equal cell go wrong: cells
+of every population around its steps of 4, chunks of 16, batches of 64 and
+sub-batches of 16 and 32 particles (empty ones among them), on a grid whose
+extents are no multiple of a brick; particles that moved to neighbouring
+cells after the binning; and values that are not finite, which must reach the
+stencil nodes of their particle and no other node.  Against the oracle at the
+tolerances of the other interpolation tests (FP64 1e-12, FP32-mixed 1e-5
+relative L2)."""
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_interpolation import P2G_FACTORY, P2G_SHAPE, TOL, rel_l2, shaped
+
+pytestmark = pytest.mark.gpu
+
+POPULATION = [0, 1, 2, 3, 4, 5, 7, 8, 9, 0, 12, 13, 15, 16, 17, 20, 31, 32, 33, 48, 63, 64, 65,
+              0, 0, 130]
+CELLS = (5, 7, 19)
+CELL = 0.5
+LOW = np.array([0.25, -1.0, 2.0])
+SETS = [(0, 1, 4), (0, 1), (0,), (1,), (2,), (3,), (4,)]
+
+
+class Cloud:
+    def __init__(self, ca, oracle, seed, moved=0.0):
+        rng = np.random.default_rng(seed)
+        cells = np.stack(np.meshgrid(*[np.arange(c) for c in CELLS], indexing="ij"), -1)
+        cells = cells.reshape(-1, 3)
+        pop = np.resize(POPULATION, len(cells))
+        cell_of = np.repeat(cells, pop, axis=0)
+        self.n = len(cell_of)
+        high = LOW + CELL * np.array(CELLS)
+        pts = LOW + CELL * (cell_of + rng.uniform(0.0, 1.0, size=(self.n, 3)))
+        gm = ca.createUniformGlobalMesh(LOW, high, CELL)
+        self.lg = ca.createLocalGrid(ca.createGlobalGrid(gm, [True] * 3), 1)
+        self.mesh = oracle.OMesh(LOW, high, CELL, halo=1)
+        t = torch.tensor(pts, device="cuda")
+        self.bins = ca.createLinkedCellList(t, [CELL] * 3, LOW, high)
+        pts = pts[self.bins.permutes.cpu().numpy()]
+        if moved:
+            pts = pts + moved * CELL * rng.normal(size=pts.shape)
+            pts = LOW + np.mod(pts - LOW, high - LOW)
+        self.pts_np = pts
+        self.pts = torch.tensor(pts, device="cuda")
+        self.values = {op: rng.normal(size=(self.n, P2G_SHAPE[op][0])) for op in range(5)}
+
+    def p2g(self, ca, ops, order, dtype):
+        arrays, fs = [], []
+        for op in ops:
+            layout = ca.createArrayLayout(self.lg, P2G_SHAPE[op][1], ca.Node())
+            arrays.append(ca.createArray("g", layout, dtype=dtype))
+            v = torch.tensor(shaped(self.values[op], P2G_SHAPE[op][0]), dtype=dtype, device="cuda")
+            fs.append(getattr(ca, P2G_FACTORY[op])(v, -0.75))
+        halo = ca.createHalo(ca.NodeHaloPattern(), 1, arrays[0])
+        ca.p2g(fs, self.pts, self.n, ca.Spline(order), halo, arrays, bins=self.bins)
+        assert ca.check_domain() == 0
+        return [a.view().cpu().numpy() for a in arrays]
+
+    def reference(self, oracle, op, order, dtype):
+        ref = self.mesh.grid(P2G_SHAPE[op][1])
+        v = self.values[op]
+        if dtype == torch.float32:
+            v = v.astype(np.float32).astype(np.float64)
+        oracle.p2g(self.mesh, order, op, -0.75, self.pts_np, v, ref)
+        return ref
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("moved", [0.0, 0.4])
+def test_group_sizes(ca, oracle, order, dtype, moved):
+    c = Cloud(ca, oracle, 31 + order, moved)
+    own = c.mesh.owned_slices()
+    ref = {op: c.reference(oracle, op, order, dtype) for op in range(5)}
+    for ops in SETS:
+        for op, got in zip(ops, c.p2g(ca, ops, order, dtype)):
+            assert rel_l2(got[own], ref[op][own]) < TOL[dtype], (ops, op)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("order", [1, 2, 3])
+def test_values_that_are_not_finite(ca, oracle, order, dtype):
+    c = Cloud(ca, oracle, 77 + order)
+    bad = [np.inf, -np.inf, np.nan]
+    for op, at in ((0, 11), (1, 700), (4, 1500)):
+        for k, b in enumerate(bad):
+            c.values[op][at + 400 * k, -1] = b
+    own = c.mesh.owned_slices()
+    with np.errstate(all="ignore"):
+        for op, got in zip((0, 1, 4), c.p2g(ca, (0, 1, 4), order, dtype)):
+            ref = c.reference(oracle, op, order, dtype)[own]
+            fine = np.isfinite(ref)
+            assert not fine.all() and fine.mean() > 0.3
+            assert np.array_equal(fine, np.isfinite(got[own]))
+            assert rel_l2(got[own][fine], ref[fine]) < TOL[dtype]
