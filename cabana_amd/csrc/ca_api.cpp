@@ -459,6 +459,49 @@ cabana_amd_status make_gfield( cabana_amd_context* ctx, const MeshDev& m,
     return CABANA_AMD_OK;
 }
 
+// Bytes from a grid's first element to its last.
+size_t grid_span( const GFieldDev& g, bool fp64 )
+{
+    int64_t last = 0;
+    for ( int d = 0; d < 4; ++d )
+        last += (int64_t)( g.ext[d] - 1 ) * g.s[d];
+    return (size_t)( last + 1 ) * ( fp64 ? 8 : 4 );
+}
+bool grids_overlap( const GFieldDev& x, const GFieldDev& y, bool fp64 )
+{
+    return x.data < y.data + grid_span( y, fp64 ) && y.data < x.data + grid_span( x, fp64 );
+}
+
+// Applies a halo launch to every distinct grid of a call once, in call order:
+// grids whose memory does not overlap go into one launch, one that overlaps an
+// earlier one starts the next.
+template <class F>
+hipError_t halo_over( const GFieldDev* grids, int n, bool fp64, F&& launch )
+{
+    GFieldDev batch[MAX_CALL_TERMS];
+    int nb = 0;
+    hipError_t e = hipSuccess;
+    for ( int i = 0; i < n && e == hipSuccess; ++i )
+    {
+        if ( !grids[i].data )
+            continue;
+        bool seen = false, overlap = false;
+        for ( int j = 0; j < i; ++j )
+            seen = seen || grids[j].data == grids[i].data;
+        if ( seen )
+            continue;
+        for ( int j = 0; j < nb; ++j )
+            overlap = overlap || grids_overlap( batch[j], grids[i], fp64 );
+        if ( overlap )
+        {
+            e = launch( batch, nb );
+            nb = 0;
+        }
+        batch[nb++] = grids[i];
+    }
+    return e == hipSuccess && nb > 0 ? launch( batch, nb ) : e;
+}
+
 bool same_grid( const GFieldDev& a, const GFieldDev& b )
 {
     return a.data == b.data && a.s[0] == b.s[0] && a.s[1] == b.s[1] &&
@@ -1174,13 +1217,11 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     int32_t* hist = reinterpret_cast<int32_t*>( digit_base + nhist + 64 );
     int64_t* sums = static_cast<int64_t*>( ctx->scratch[SLOT_SCAN] );
     CA_HIP( ctx, launch_auto_bin_keys( *ctx, pts, n, m, keys, s ), "bin keys" );
-    int32_t* sorted = keys;
     CA_HIP( ctx,
             launch_lcl_sort( *ctx, n, key_bits, keys, keys + nkey, keys + 2 * nkey,
-                             keys + 3 * nkey, hist, digit_base, sums, nblock, perm, 0, &sorted,
-                             s ),
+                             keys + 3 * nkey, hist, digit_base, sums, nblock, perm, 0, ncell,
+                             counts, offsets, s ),
             "bin sort" );
-    CA_HIP( ctx, launch_lcl_bounds( *ctx, sorted, n, ncell, counts, offsets, s ), "bin bounds" );
     ctx->auto_bins = {};
     ctx->auto_bins.counts = counts;
     ctx->auto_bins.offsets = offsets;
@@ -1457,16 +1498,13 @@ cabana_amd_status p2g_impl( cabana_amd_context* ctx, const cabana_amd_mesh* mesh
         }
     }
     // Fold every distinct grid once.
+    GFieldDev grids[MAX_CALL_TERMS];
     for ( int i = 0; i < num_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || T[j].grid.data == T[i].grid.data;
-        if ( !seen )
-            CA_HIP( ctx,
-                    launch_halo_scatter_sum( *ctx, fp64, m, T[i].grid, w, s ),
-                    "halo scatter" );
-    }
+        grids[i] = T[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_scatter_sum( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo scatter" );
     return CABANA_AMD_OK;
 }
 } // namespace
@@ -1623,15 +1661,13 @@ extern "C" cabana_amd_status cabana_amd_g2p(
     }
     hipStream_t s = static_cast<hipStream_t>( stream );
     CA_CHECK( auto_bins( ctx, m, order, a.points, n, bins, s ) );
+    GFieldDev grids[MAX_CALL_TERMS];
     for ( int i = 0; i < num_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || T[j].grid.data == T[i].grid.data;
-        if ( !seen )
-            CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, T[i].grid, w, s ),
-                    "halo gather" );
-    }
+        grids[i] = T[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_gather( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo gather" );
     if ( n <= 0 )
         return CABANA_AMD_OK;
     return g2p_passes( ctx, order, fp64, a, T.data(), num_terms, n, bins, s );
@@ -1644,18 +1680,7 @@ extern "C" cabana_amd_status cabana_amd_g2p(
 namespace
 {
 // Bytes from a grid's first element to one past its last.
-size_t grid_span( const GFieldDev& g, bool fp64 )
-{
-    int64_t last = 0;
-    for ( int d = 0; d < 4; ++d )
-        last += (int64_t)( g.ext[d] - 1 ) * g.s[d];
-    return (size_t)( last + 1 ) * ( fp64 ? 8 : 4 );
-}
 
-bool grids_overlap( const GFieldDev& x, const GFieldDev& y, bool fp64 )
-{
-    return x.data < y.data + grid_span( y, fp64 ) && y.data < x.data + grid_span( x, fp64 );
-}
 } // namespace
 
 extern "C" cabana_amd_status cabana_amd_g2p2g(
@@ -1749,14 +1774,13 @@ extern "C" cabana_amd_status cabana_amd_g2p2g(
     hipStream_t s = static_cast<hipStream_t>( stream );
     // Halo::gather of every distinct G2P grid (Cabana_Grid_Interpolation
     // Performance.cpp:140-141 gathers before the point loop).
+    GFieldDev grids[MAX_CALL_TERMS];
     for ( int i = 0; i < num_g2p_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || a.g[j].grid.data == a.g[i].grid.data;
-        if ( !seen )
-            CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, a.g[i].grid, w, s ), "halo gather" );
-    }
+        grids[i] = a.g[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_g2p_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_gather( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo gather" );
     if ( n > 0 )
     {
         // A G2P grid that a P2G term also adds into is read from a copy
@@ -1804,14 +1828,11 @@ extern "C" cabana_amd_status cabana_amd_g2p2g(
     }
     // Halo::scatter(Sum) of every distinct P2G grid.
     for ( int i = 0; i < num_p2g_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || a.s[j].grid.data == a.s[i].grid.data;
-        if ( !seen )
-            CA_HIP( ctx, launch_halo_scatter_sum( *ctx, fp64, m, a.s[i].grid, w, s ),
-                    "halo scatter" );
-    }
+        grids[i] = a.s[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_p2g_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_scatter_sum( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo scatter" );
     return CABANA_AMD_OK;
 }
 
@@ -1883,16 +1904,13 @@ cabana_amd_status p2g_adjoint_impl( cabana_amd_context* ctx, const cabana_amd_me
     }
     hipStream_t s = static_cast<hipStream_t>( stream );
     CA_CHECK( auto_bins( ctx, m, order, a.points, n, bins, s ) );
+    GFieldDev grids[MAX_CALL_TERMS];
     for ( int i = 0; i < num_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || T[j].grid.data == T[i].grid.data;
-        if ( !seen )
-            CA_HIP( ctx,
-                    launch_halo_adjoint_fill( *ctx, fp64, m, T[i].grid, w, s ),
-                    "halo adjoint fill" );
-    }
+        grids[i] = T[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_adjoint_fill( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo adjoint fill" );
     if ( n <= 0 )
         return CABANA_AMD_OK;
     const bool mpm = num_terms == 3 && xbar && T[0].form == FORM_SV &&
@@ -1925,7 +1943,7 @@ cabana_amd_status p2g_adjoint_impl( cabana_amd_context* ctx, const cabana_amd_me
         if ( own_grid )
         {
             // Forward ghost fill of the grid read for the position cotangent.
-            CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, X[0].grid, w, s ), "halo gather" );
+            CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, &X[0].grid, 1, w, s ), "halo gather" );
             a.nterms = 5;
             for ( int i = 0; i < 3; ++i )
                 a.t[i] = T[i];
@@ -2058,27 +2076,23 @@ extern "C" cabana_amd_status cabana_amd_g2p_adjoint(
     hipStream_t s = static_cast<hipStream_t>( stream );
     CA_CHECK( auto_bins( ctx, m, order, a.points, n, bins, s ) );
     // Forward ghost fill of the grids read for the position cotangent.
+    GFieldDev grids[MAX_CALL_TERMS];
     if ( xbar )
+    {
         for ( int i = 0; i < num_terms; ++i )
-        {
-            bool seen = false;
-            for ( int j = 0; j < i; ++j )
-                seen = seen || T[j].gx.data == T[i].gx.data;
-            if ( !seen )
-                CA_HIP( ctx,
-                        launch_halo_gather( *ctx, fp64, m, T[i].gx, w, s ),
-                        "halo gather" );
-        }
+            grids[i] = T[i].gx;
+        CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                    return launch_halo_gather( *ctx, fp64, m, g, ng, w, s );
+                } ),
+                "halo gather" );
+    }
     // Cotangent grids: clear ghosts, scatter, fold.
     for ( int i = 0; i < num_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || T[j].grid.data == T[i].grid.data;
-        if ( !seen && T[i].grid.data )
-            CA_HIP( ctx, launch_zero_ghosts( *ctx, fp64, m, T[i].grid, s ),
-                    "zero ghosts" );
-    }
+        grids[i] = T[i].grid;
+    CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_zero_ghosts( *ctx, fp64, m, g, ng, s );
+            } ),
+            "zero ghosts" );
     if ( n > 0 && xbar )
     {
         // Position cotangents: a G2P-shaped gather of the forward grid,
@@ -2154,16 +2168,10 @@ extern "C" cabana_amd_status cabana_amd_g2p_adjoint(
             }
         }
     }
-    for ( int i = 0; i < num_terms; ++i )
-    {
-        bool seen = false;
-        for ( int j = 0; j < i; ++j )
-            seen = seen || T[j].grid.data == T[i].grid.data;
-        if ( !seen && T[i].grid.data )
-            CA_HIP( ctx,
-                    launch_halo_scatter_sum( *ctx, fp64, m, T[i].grid, w, s ),
-                    "halo scatter" );
-    }
+    CA_HIP( ctx, halo_over( grids, num_terms, fp64, [&]( const GFieldDev* g, int ng ) {
+                return launch_halo_scatter_sum( *ctx, fp64, m, g, ng, w, s );
+            } ),
+            "halo scatter" );
     return CABANA_AMD_OK;
 }
 
@@ -2203,7 +2211,7 @@ extern "C" cabana_amd_status cabana_amd_halo_gather(
     bool fp64;
     CA_CHECK( halo_common( ctx, mesh, grid, halo_width, m, g, w, fp64 ) );
     CA_HIP( ctx,
-            launch_halo_gather( *ctx, fp64, m, g, w,
+            launch_halo_gather( *ctx, fp64, m, &g, 1, w,
                                 static_cast<hipStream_t>( stream ) ),
             "halo gather" );
     return CABANA_AMD_OK;
@@ -2221,7 +2229,7 @@ extern "C" cabana_amd_status cabana_amd_halo_scatter_sum(
     bool fp64;
     CA_CHECK( halo_common( ctx, mesh, grid, halo_width, m, g, w, fp64 ) );
     CA_HIP( ctx,
-            launch_halo_scatter_sum( *ctx, fp64, m, g, w,
+            launch_halo_scatter_sum( *ctx, fp64, m, &g, 1, w,
                                      static_cast<hipStream_t>( stream ) ),
             "halo scatter" );
     return CABANA_AMD_OK;
@@ -2331,14 +2339,11 @@ extern "C" cabana_amd_status cabana_amd_linked_cell_build(
             launch_lcl_keys( *ctx, pos, begin, end, g, (int32_t)ncell, keys,
                              ctx->bad, s ),
             "bin keys" );
-    int32_t* sorted = keys;
     CA_HIP( ctx,
             launch_lcl_sort( *ctx, np, key_bits, keys, keys + nkey,
                              keys + 2 * nkey, keys + 3 * nkey, hist, digit_base,
-                             sums, nblock, permutes, begin, &sorted, s ),
+                             sums, nblock, permutes, begin, ncell, counts, offsets, s ),
             "bin sort" );
-    CA_HIP( ctx, launch_lcl_bounds( *ctx, sorted, np, ncell, counts, offsets, s ),
-            "bin bounds" );
     // The reference fences after each phase; one wait here reports
     // particles outside the grid.
     unsigned long long bad = 0;
@@ -2464,7 +2469,7 @@ extern "C" cabana_amd_status cabana_amd_bov_write_time_step(
     for ( int d = 0; d < 3; ++d )
         any_periodic = any_periodic || m.periodic[d];
     if ( node && gather_array && any_periodic )
-        CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, g, 0, s ), "halo gather" );
+        CA_HIP( ctx, launch_halo_gather( *ctx, fp64, m, &g, 1, 0, s ), "halo gather" );
     const int dofs = grid->extent[3];
     const size_t es = fp64 ? 8 : 4;
     const size_t count = (size_t)n[0] * n[1] * n[2] * dofs;

@@ -17,7 +17,7 @@ inline dim3 blocks_for( int64_t n )
 // Owned entity range of one dimension on one rank
 // (Cabana_Grid_LocalGrid_impl.hpp:239-280, 430-450, 534-560): N entities,
 // plus the closing boundary node in a non-periodic node-centred dimension.
-__device__ __forceinline__ int owned_hi( const MeshDev& m, int d )
+__host__ __device__ __forceinline__ int owned_hi( const MeshDev& m, int d )
 {
     return m.halo + m.num_cell[d] + ( ( m.periodic[d] || m.stag[d] ) ? 0 : 1 );
 }
@@ -46,36 +46,97 @@ __device__ __forceinline__ int owner_of( const MeshDev& m, int d, int x, int w,
     return -1;
 }
 
-template <class Real>
-__global__ __launch_bounds__( BLOCK ) void halo_fill_kernel( MeshDev m,
-                                                             GFieldDev g,
-                                                             int w,
-                                                             int zero_other )
+// The grids of one halo launch (blockIdx.y picks one).
+constexpr int HALO_GRIDS = 4;
+struct HaloGrids
 {
-    const int64_t n = (int64_t)g.ext[0] * g.ext[1] * g.ext[2];
+    GFieldDev g[HALO_GRIDS];
+};
+
+// One dimension of a box whose shell a halo kernel walks: positions
+// [lo, lo + n), of which the first `head` and the last `tail` (head + tail <=
+// n) are shell positions and the others interior.
+struct ShellDim
+{
+    int lo;
+    int n;
+    int head;
+    int tail;
+    __device__ int shell() const { return head + tail; }
+    __device__ int inner() const { return n - head - tail; }
+    __device__ int shell_at( int i ) const { return lo + ( i < head ? i : n - tail + ( i - head ) ); }
+    __device__ int inner_at( int i ) const { return lo + head + i; }
+};
+
+// Nodes of a box with a shell position in some dimension, numbered slab by
+// slab: shell x all x all, interior x shell x all, interior x interior x
+// shell.  Only these are visited: over the whole 131^3 grid the fold took
+// 22 us, over its shell 5 us.
+struct Shell
+{
+    ShellDim d[3];
+    __host__ __device__ int64_t size() const
+    {
+        const int64_t n1 = d[1].n, n2 = d[2].n;
+        const int64_t s0 = d[0].head + d[0].tail, s1 = d[1].head + d[1].tail,
+                      s2 = d[2].head + d[2].tail;
+        return s0 * n1 * n2 + ( d[0].n - s0 ) * ( s1 * n2 + ( n1 - s1 ) * s2 );
+    }
+    __device__ void at( int e, int x[3] ) const
+    {
+        const int a = d[0].shell() * d[1].n * d[2].n;
+        if ( e < a )
+        {
+            x[0] = d[0].shell_at( e / ( d[1].n * d[2].n ) );
+            x[1] = d[1].lo + e / d[2].n % d[1].n;
+            x[2] = d[2].lo + e % d[2].n;
+            return;
+        }
+        e -= a;
+        const int b = d[0].inner() * d[1].shell() * d[2].n;
+        if ( e < b )
+        {
+            x[0] = d[0].inner_at( e / ( d[1].shell() * d[2].n ) );
+            x[1] = d[1].shell_at( e / d[2].n % d[1].shell() );
+            x[2] = d[2].lo + e % d[2].n;
+            return;
+        }
+        e -= b;
+        x[0] = d[0].inner_at( e / ( d[1].inner() * d[2].shell() ) );
+        x[1] = d[1].inner_at( e / d[2].shell() % d[1].inner() );
+        x[2] = d[2].shell_at( e % d[2].shell() );
+    }
+};
+
+// Fill: every ghost node takes its owner's value; one that no message reaches
+// is zeroed (zero_other) or left.  With owners == false every ghost is zeroed.
+template <class Real>
+__global__ __launch_bounds__( BLOCK ) void halo_fill_kernel( MeshDev m, HaloGrids gs, Shell shell,
+                                                             int w, int zero_other, int owners )
+{
     const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( e >= n )
+    if ( e >= shell.size() )
         return;
-    const int i = (int)( e / ( (int64_t)g.ext[1] * g.ext[2] ) );
-    const int j = (int)( ( e / g.ext[2] ) % g.ext[1] );
-    const int k = (int)( e % g.ext[2] );
-    bool gi, gj, gk;
-    const int oi = owner_of( m, 0, i, w, gi );
-    const int oj = owner_of( m, 1, j, w, gj );
-    const int ok = owner_of( m, 2, k, w, gk );
-    if ( !gi && !gj && !gk )
-        return; // owned
-    Real* dst = gptr<Real>( g, i * g.s[0] + j * g.s[1] +
-                k * g.s[2] );
-    if ( oi < 0 || oj < 0 || ok < 0 )
+    const GFieldDev& g = gs.g[blockIdx.y];
+    int x[3], o[3];
+    shell.at( (int)e, x );
+    bool reached = owners != 0;
+#pragma unroll
+    for ( int d = 0; d < 3; ++d )
+    {
+        bool ghost;
+        o[d] = owner_of( m, d, x[d], w, ghost );
+        reached = reached && o[d] >= 0;
+    }
+    Real* dst = gptr<Real>( g, x[0] * g.s[0] + x[1] * g.s[1] + x[2] * g.s[2] );
+    if ( !reached )
     {
         if ( zero_other )
             for ( int d = 0; d < g.ext[3]; ++d )
                 dst[d * g.s[3]] = Real( 0 );
         return;
     }
-    const Real* src = gptr<const Real>( g, oi * g.s[0] +
-                      oj * g.s[1] + ok * g.s[2] );
+    const Real* src = gptr<const Real>( g, o[0] * g.s[0] + o[1] * g.s[1] + o[2] * g.s[2] );
     for ( int d = 0; d < g.ext[3]; ++d )
         dst[d * g.s[3]] = src[d * g.s[3]];
 }
@@ -84,26 +145,16 @@ __global__ __launch_bounds__( BLOCK ) void halo_fill_kernel( MeshDev m,
 // gathers its images itself, so the sum needs no atomics and its order is
 // fixed (the reference's MPI Waitany order is not).
 template <class Real>
-__global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m,
-                                                             GFieldDev g,
+__global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m, HaloGrids gs, Shell shell,
                                                              int w )
 {
-    int lo[3], n[3];
-#pragma unroll
-    for ( int d = 0; d < 3; ++d )
-    {
-        lo[d] = m.halo;
-        n[d] = owned_hi( m, d ) - m.halo;
-    }
-    const int64_t total = (int64_t)n[0] * n[1] * n[2];
     const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( e >= total )
+    if ( e >= shell.size() )
         return;
-    const int x[3] = { lo[0] + (int)( e / ( (int64_t)n[1] * n[2] ) ),
-                       lo[1] + (int)( ( e / n[2] ) % n[1] ),
-                       lo[2] + (int)( e % n[2] ) };
+    const GFieldDev& g = gs.g[blockIdx.y];
+    int x[3];
+    shell.at( (int)e, x );
     int cand[3][3], nc[3];
-    bool any = false;
 #pragma unroll
     for ( int d = 0; d < 3; ++d )
     {
@@ -117,10 +168,7 @@ __global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m,
             if ( x[d] >= h + N - w )
                 cand[d][nc[d]++] = x[d] - N;
         }
-        any = any || nc[d] > 1;
     }
-    if ( !any )
-        return;
     Real* dst = gptr<Real>( g, x[0] * g.s[0] +
                 x[1] * g.s[1] + x[2] * g.s[2] );
     for ( int d = 0; d < g.ext[3]; ++d )
@@ -138,29 +186,6 @@ __global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m,
                 }
         dst[d * g.s[3]] += acc;
     }
-}
-
-template <class Real>
-__global__ __launch_bounds__( BLOCK ) void zero_ghosts_kernel( MeshDev m,
-                                                               GFieldDev g )
-{
-    const int64_t n = (int64_t)g.ext[0] * g.ext[1] * g.ext[2];
-    const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( e >= n )
-        return;
-    const int x[3] = { (int)( e / ( (int64_t)g.ext[1] * g.ext[2] ) ),
-                       (int)( ( e / g.ext[2] ) % g.ext[1] ),
-                       (int)( e % g.ext[2] ) };
-    bool owned = true;
-#pragma unroll
-    for ( int d = 0; d < 3; ++d )
-        owned = owned && x[d] >= m.halo && x[d] < owned_hi( m, d );
-    if ( owned )
-        return;
-    Real* dst = gptr<Real>( g, x[0] * g.s[0] +
-                x[1] * g.s[1] + x[2] * g.s[2] );
-    for ( int d = 0; d < g.ext[3]; ++d )
-        dst[d * g.s[3]] = Real( 0 );
 }
 
 // ---------------------------------------------------------------------------
@@ -231,32 +256,51 @@ __global__ __launch_bounds__( SCAN_BLOCK ) void scan_reduce_kernel(
     }
 }
 
+// Exclusive scan of one value per thread over a workgroup of SCAN_BLOCK
+// threads; returns the prefix of this thread and leaves the total in *total.
+template <class T>
+__device__ __forceinline__ T scan_group( T v, T* wsum, T* total )
+{
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    T x = v;
+#pragma unroll
+    for ( int o = 1; o < 64; o <<= 1 )
+    {
+        const T u = __shfl_up( x, o, 64 );
+        if ( lane >= o )
+            x += u;
+    }
+    if ( lane == 63 )
+        wsum[wv] = x;
+    __syncthreads();
+    T before = 0, all = 0;
+#pragma unroll
+    for ( int q = 0; q < SCAN_BLOCK / 64; ++q )
+    {
+        const T s = wsum[q];
+        before += q < wv ? s : T( 0 );
+        all += s;
+    }
+    // wsum is free for the next scan.
+    __syncthreads();
+    *total = all;
+    return before + x - v;
+}
+
 // Exclusive scan of the block sums by one workgroup (sequential per thread
 // chunk, then a workgroup scan of the chunk totals).
 __global__ __launch_bounds__( SCAN_BLOCK ) void scan_block_sums_kernel(
     int64_t* block_sums, int64_t nb )
 {
-    __shared__ int64_t part[SCAN_BLOCK];
+    __shared__ int64_t wsum[SCAN_BLOCK / 64];
     const int64_t chunk = ( nb + SCAN_BLOCK - 1 ) / SCAN_BLOCK;
     const int64_t lo = threadIdx.x * chunk;
     const int64_t hi = lo + chunk < nb ? lo + chunk : nb;
     int64_t s = 0;
     for ( int64_t i = lo; i < hi; ++i )
         s += block_sums[i];
-    part[threadIdx.x] = s;
-    __syncthreads();
-    if ( threadIdx.x == 0 )
-    {
-        int64_t run = 0;
-        for ( int t = 0; t < SCAN_BLOCK; ++t )
-        {
-            const int64_t v = part[t];
-            part[t] = run;
-            run += v;
-        }
-    }
-    __syncthreads();
-    int64_t run = part[threadIdx.x];
+    int64_t total;
+    int64_t run = scan_group( s, wsum, &total );
     for ( int64_t i = lo; i < hi; ++i )
     {
         const int64_t v = block_sums[i];
@@ -265,37 +309,70 @@ __global__ __launch_bounds__( SCAN_BLOCK ) void scan_block_sums_kernel(
     }
 }
 
+// Exclusive scan of up to SCAN_ONE values by one workgroup, SCAN_ITEMS
+// consecutive values a thread at a time, each round's reads issued before the
+// round before it is scanned.  A single workgroup is bound by the latency of
+// its rounds (about 1 us each), the three-kernel scan by its launches: 16384
+// values take 5 us against 21 us, and the two meet above 65536.
+constexpr int SCAN_ITEMS = 8;
+constexpr int64_t SCAN_ONE = 65536;
+template <class F>
+__device__ __forceinline__ int64_t scan_one( const int32_t* in, int64_t n, F&& put )
+{
+    __shared__ int64_t wsum[SCAN_BLOCK / 64];
+    const int64_t step = SCAN_BLOCK * SCAN_ITEMS;
+    int32_t next[SCAN_ITEMS];
+    auto read = [&]( int64_t base ) {
+#pragma unroll
+        for ( int k = 0; k < SCAN_ITEMS; ++k )
+        {
+            const int64_t i = base + (int64_t)threadIdx.x * SCAN_ITEMS + k;
+            next[k] = i < n ? in[i] : 0;
+        }
+    };
+    int64_t carry = 0;
+    read( 0 );
+    for ( int64_t base = 0; base < n; base += step )
+    {
+        int32_t v[SCAN_ITEMS];
+        int64_t sum = 0;
+#pragma unroll
+        for ( int k = 0; k < SCAN_ITEMS; ++k )
+        {
+            v[k] = next[k];
+            sum += v[k];
+        }
+        read( base + step );
+        int64_t total;
+        int64_t run = carry + scan_group( sum, wsum, &total );
+#pragma unroll
+        for ( int k = 0; k < SCAN_ITEMS; ++k )
+        {
+            const int64_t i = base + (int64_t)threadIdx.x * SCAN_ITEMS + k;
+            if ( i < n )
+                put( i, v[k], run );
+            run += v[k];
+        }
+        carry += total;
+    }
+    return carry;
+}
+
+__global__ __launch_bounds__( SCAN_BLOCK ) void scan_one_kernel( const int32_t* in, int64_t* out,
+                                                                 int64_t n )
+{
+    scan_one( in, n, [&]( int64_t i, int32_t, int64_t before ) { out[i] = before; } );
+}
+
 __global__ __launch_bounds__( SCAN_BLOCK ) void scan_apply_kernel(
     const int32_t* in, int64_t* out, int64_t n, const int64_t* block_sums )
 {
     __shared__ int64_t wsum[SCAN_BLOCK / 64];
     const int64_t i = (int64_t)blockIdx.x * SCAN_BLOCK + threadIdx.x;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int64_t x = ( i < n ) ? in[i] : 0;
-    // Inclusive wave scan.
-    int64_t v = x;
-    for ( int o = 1; o < 64; o <<= 1 )
-    {
-        const int64_t u = __shfl_up( v, o, 64 );
-        if ( lane >= o )
-            v += u;
-    }
-    if ( lane == 63 )
-        wsum[wv] = v;
-    __syncthreads();
-    if ( threadIdx.x == 0 )
-    {
-        int64_t run = 0;
-        for ( int w = 0; w < SCAN_BLOCK / 64; ++w )
-        {
-            const int64_t t = wsum[w];
-            wsum[w] = run;
-            run += t;
-        }
-    }
-    __syncthreads();
+    int64_t total;
+    const int64_t before = scan_group( i < n ? (int64_t)in[i] : 0, wsum, &total );
     if ( i < n )
-        out[i] = block_sums[blockIdx.x] + wsum[wv] + v - x;
+        out[i] = block_sums[blockIdx.x] + before;
 }
 
 // ---------------------------------------------------------------------------
@@ -512,6 +589,153 @@ __global__ __launch_bounds__( BLOCK ) void lcl_bounds_kernel(
     counts[c] = (int32_t)( hi - lo );
 }
 
+// The whole sort of up to RS_SMALL_BLOCK * ITEMS keys by one workgroup: every
+// pass stays in LDS (keys, 16-bit indices, per-wave digit counts), with the
+// ranks of radix_scatter_kernel; then the permutation and, for up to
+// RS_SMALL_CELLS bins, counts and offsets by binary search of the keys in LDS.
+// At these sizes the launches of the tiled sort (three a pass) and of the
+// bounds are what a build costs: 4096 particles in 512 cells take 13 us
+// against 100 us.
+constexpr int RS_SMALL_BLOCK = 1024;
+constexpr int RS_SMALL_WAVES = RS_SMALL_BLOCK / 64;
+constexpr int64_t RS_SMALL_CELLS = 16384;
+constexpr int64_t RS_SMALL_MAX = RS_SMALL_BLOCK * 16;
+
+template <int ITEMS>
+constexpr size_t rs_small_lds()
+{
+    return RS_SMALL_BLOCK * ITEMS * ( sizeof( int32_t ) + sizeof( uint16_t ) ) +
+           sizeof( uint32_t ) * RS_SMALL_WAVES * RS_MAX_BINS;
+}
+
+template <int ITEMS>
+__global__ __launch_bounds__( RS_SMALL_BLOCK ) void lcl_sort_small_kernel(
+    const int32_t* keys, int n, int passes, int dbits, int64_t* permutes, int64_t begin,
+    int32_t* sorted, int64_t ncell, int32_t* counts, int64_t* offsets )
+{
+    extern __shared__ __align__( 16 ) unsigned char smem[];
+    int32_t* lkey = reinterpret_cast<int32_t*>( smem );
+    uint32_t( *wcnt )[RS_MAX_BINS] =
+        reinterpret_cast<uint32_t( * )[RS_MAX_BINS]>( lkey + RS_SMALL_BLOCK * ITEMS );
+    uint16_t* lval = reinterpret_cast<uint16_t*>( wcnt + RS_SMALL_WAVES );
+    __shared__ uint32_t wsum[RS_MAX_BINS / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t below = ( 1ull << lane ) - 1ull;
+    const int wbase = w * 64 * ITEMS;
+    const uint32_t mask = ( 1u << dbits ) - 1u;
+    int32_t key[ITEMS];
+    uint16_t val[ITEMS];
+#pragma unroll
+    for ( int k = 0; k < ITEMS; ++k )
+    {
+        const int i = wbase + k * 64 + lane;
+        key[k] = i < n ? keys[i] : 0;
+        val[k] = (uint16_t)i;
+    }
+    for ( int p = 0; p < passes; ++p )
+    {
+        const int shift = p * dbits;
+        for ( int c = lane; c < RS_MAX_BINS; c += 64 )
+            wcnt[w][c] = 0;
+        __syncthreads();
+        uint32_t rank[ITEMS];
+#pragma unroll
+        for ( int k = 0; k < ITEMS; ++k )
+        {
+            const bool ok = wbase + k * 64 + lane < n;
+            const uint32_t d = ( (uint32_t)key[k] >> shift ) & mask;
+            uint64_t peers = __ballot( ok );
+#pragma unroll
+            for ( int b = 0; b < RS_MAX_BITS; ++b )
+            {
+                const bool set = ( d >> b ) & 1u;
+                const uint64_t bb = __ballot( set );
+                peers &= set ? bb : ~bb;
+            }
+            if ( ok )
+            {
+                const uint32_t c = wcnt[w][d];
+                rank[k] = c + (uint32_t)__popcll( peers & below );
+                if ( ( peers >> lane ) == 1ull )
+                    wcnt[w][d] = c + (uint32_t)__popcll( peers );
+            }
+        }
+        __syncthreads();
+        // Per digit (one thread each): prefix over the waves, then over the
+        // digits; wcnt becomes the first output position of (wave, digit).
+        uint32_t run = 0, x = 0;
+        if ( threadIdx.x < RS_MAX_BINS )
+        {
+            for ( int q = 0; q < RS_SMALL_WAVES; ++q )
+            {
+                const uint32_t c = wcnt[q][threadIdx.x];
+                wcnt[q][threadIdx.x] = run;
+                run += c;
+            }
+            x = run;
+#pragma unroll
+            for ( int o = 1; o < 64; o <<= 1 )
+            {
+                const uint32_t u = __shfl_up( x, o, 64 );
+                if ( lane >= o )
+                    x += u;
+            }
+            if ( lane == 63 )
+                wsum[w] = x;
+        }
+        __syncthreads();
+        if ( threadIdx.x < RS_MAX_BINS )
+        {
+            uint32_t start = x - run;
+            for ( int q = 0; q < w; ++q )
+                start += wsum[q];
+            for ( int q = 0; q < RS_SMALL_WAVES; ++q )
+                wcnt[q][threadIdx.x] += start;
+        }
+        __syncthreads();
+#pragma unroll
+        for ( int k = 0; k < ITEMS; ++k )
+            if ( wbase + k * 64 + lane < n )
+            {
+                const uint32_t d = ( (uint32_t)key[k] >> shift ) & mask;
+                const uint32_t at = wcnt[w][d] + rank[k];
+                lkey[at] = key[k];
+                lval[at] = val[k];
+            }
+        __syncthreads();
+#pragma unroll
+        for ( int k = 0; k < ITEMS; ++k )
+        {
+            const int i = wbase + k * 64 + lane;
+            if ( i < n )
+            {
+                key[k] = lkey[i];
+                val[k] = lval[i];
+            }
+        }
+    }
+    const bool bounds = ncell <= RS_SMALL_CELLS;
+#pragma unroll
+    for ( int k = 0; k < ITEMS; ++k )
+    {
+        const int i = wbase + k * 64 + lane;
+        if ( i < n )
+        {
+            permutes[i] = begin + val[k];
+            if ( !bounds )
+                sorted[i] = key[k];
+        }
+    }
+    if ( bounds )
+        for ( int c = threadIdx.x; c < (int)ncell; c += RS_SMALL_BLOCK )
+        {
+            const int64_t lo = lower_bound_i32( lkey, n, c );
+            const int64_t hi = lower_bound_i32( lkey, n, c + 1 );
+            offsets[c] = lo;
+            counts[c] = (int32_t)( hi - lo );
+        }
+}
+
 template <class T>
 __global__ __launch_bounds__( BLOCK ) void permute_gather_kernel(
     PFieldDev f, const int64_t* permutes, int64_t begin, int64_t end,
@@ -636,28 +860,52 @@ __global__ __launch_bounds__( BLOCK ) void permute_put_words_kernel(
 // Part table of a brick tiling.  One thread per brick counts the brick's
 // particles through the cell offsets of its cell runs and the number of
 // parts of at most t.cap particles (an empty brick has none).
+// BRICK_LANES lanes sum the cell rows of a brick.
+constexpr int BRICK_LANES = 8;
 __global__ __launch_bounds__( BLOCK ) void brick_count_kernel( TileArgs t, int3 nc,
                                                                int32_t* nparts )
 {
     const int nbricks = t.ntile[0] * t.ntile[1] * t.ntile[2];
-    const int b = blockIdx.x * BLOCK + threadIdx.x;
-    if ( b >= nbricks )
-        return;
-    const int bi = b / ( t.ntile[1] * t.ntile[2] );
-    const int bj = ( b / t.ntile[2] ) % t.ntile[1];
-    const int bk = b % t.ntile[2];
-    const int i0 = bi * t.tile[0], i1 = min( i0 + t.tile[0], nc.x );
-    const int j0 = bj * t.tile[1], j1 = min( j0 + t.tile[1], nc.y );
-    const int k0 = bk * t.tile[2], k1 = min( k0 + t.tile[2], nc.z );
+    const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    const int b = (int)( e / BRICK_LANES );
+    const int sub = (int)( e % BRICK_LANES );
     int64_t count = 0;
-    for ( int i = i0; i < i1; ++i )
-        for ( int j = j0; j < j1; ++j )
+    if ( b < nbricks )
+    {
+        const int bi = b / ( t.ntile[1] * t.ntile[2] );
+        const int bj = ( b / t.ntile[2] ) % t.ntile[1];
+        const int bk = b % t.ntile[2];
+        const int i0 = bi * t.tile[0], i1 = min( i0 + t.tile[0], nc.x );
+        const int j0 = bj * t.tile[1], j1 = min( j0 + t.tile[1], nc.y );
+        const int k0 = bk * t.tile[2], k1 = min( k0 + t.tile[2], nc.z );
+        const int rows = ( i1 - i0 ) * ( j1 - j0 );
+        for ( int r = sub; r < rows; r += BRICK_LANES )
         {
+            const int i = i0 + r / ( j1 - j0 ), j = j0 + r % ( j1 - j0 );
             const int64_t first = ( (int64_t)i * nc.y + j ) * nc.z + k0;
             const int64_t last = first + ( k1 - k0 ) - 1;
             count += t.cell_offsets[last] + t.cell_counts[last] - t.cell_offsets[first];
         }
-    nparts[b] = (int32_t)( ( count + t.cap - 1 ) / t.cap );
+    }
+#pragma unroll
+    for ( int o = BRICK_LANES / 2; o > 0; o >>= 1 )
+        count += __shfl_xor( count, o, 64 );
+    if ( b < nbricks && sub == 0 )
+        nparts[b] = (int32_t)( ( count + t.cap - 1 ) / t.cap );
+}
+
+// Scan of the bricks' part counts and the part table in one launch (up to
+// SCAN_ONE bricks).
+__global__ __launch_bounds__( SCAN_BLOCK ) void part_scan_fill_kernel( const int32_t* nparts,
+                                                                       int nbricks, int2* parts,
+                                                                       int32_t* num_parts )
+{
+    const int64_t total = scan_one( nparts, nbricks, [&]( int64_t b, int32_t np, int64_t before ) {
+        for ( int q = 0; q < np; ++q )
+            parts[before + q] = make_int2( (int)b, q );
+    } );
+    if ( threadIdx.x == 0 )
+        *num_parts = (int32_t)total;
 }
 
 __global__ __launch_bounds__( BLOCK ) void part_fill_kernel( const int32_t* nparts,
@@ -820,67 +1068,111 @@ __global__ __launch_bounds__( BLOCK ) void bov_pack_kernel( GFieldDev g, int lo,
 
 } // namespace
 
-hipError_t launch_halo_gather( Launcher& L, bool fp64, const MeshDev& m,
-                               const GFieldDev& g, int width, hipStream_t s )
+namespace
 {
-    const int64_t n = (int64_t)g.ext[0] * g.ext[1] * g.ext[2];
-    L.before( "halo_gather", s );
-    if ( fp64 )
-        hipLaunchKernelGGL( halo_fill_kernel<double>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width, 0 );
-    else
-        hipLaunchKernelGGL( halo_fill_kernel<float>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width, 0 );
-    L.after( "halo_gather", s );
-    return hipGetLastError();
-}
-
-hipError_t launch_halo_adjoint_fill( Launcher& L, bool fp64, const MeshDev& m,
-                                     const GFieldDev& g, int width,
-                                     hipStream_t s )
+// The ghost nodes of the arrays, as the shell of their extents.
+Shell ghost_shell( const MeshDev& m, const GFieldDev& g )
 {
-    const int64_t n = (int64_t)g.ext[0] * g.ext[1] * g.ext[2];
-    L.before( "halo_adjoint_fill", s );
-    if ( fp64 )
-        hipLaunchKernelGGL( halo_fill_kernel<double>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width, 1 );
-    else
-        hipLaunchKernelGGL( halo_fill_kernel<float>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width, 1 );
-    L.after( "halo_adjoint_fill", s );
-    return hipGetLastError();
-}
-
-hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m,
-                                    const GFieldDev& g, int width,
-                                    hipStream_t s )
-{
-    int64_t n = 1;
+    Shell s;
     for ( int d = 0; d < 3; ++d )
-        n *= m.num_cell[d] + ( m.periodic[d] ? 0 : 1 );
-    L.before( "halo_scatter_sum", s );
-    if ( fp64 )
-        hipLaunchKernelGGL( halo_fold_kernel<double>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width );
-    else
-        hipLaunchKernelGGL( halo_fold_kernel<float>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g, width );
-    L.after( "halo_scatter_sum", s );
-    return hipGetLastError();
+    {
+        const int hi = owned_hi( m, d );
+        s.d[d] = { 0, g.ext[d], m.halo, g.ext[d] - hi };
+    }
+    return s;
 }
 
-hipError_t launch_zero_ghosts( Launcher& L, bool fp64, const MeshDev& m,
-                               const GFieldDev& g, hipStream_t s )
+// The owned nodes with periodic images in a halo of width w.
+Shell image_shell( const MeshDev& m, int w )
 {
-    const int64_t n = (int64_t)g.ext[0] * g.ext[1] * g.ext[2];
-    L.before( "zero_ghosts", s );
-    if ( fp64 )
-        hipLaunchKernelGGL( zero_ghosts_kernel<double>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g );
-    else
-        hipLaunchKernelGGL( zero_ghosts_kernel<float>, blocks_for( n ),
-                            dim3( BLOCK ), 0, s, m, g );
-    L.after( "zero_ghosts", s );
+    Shell s;
+    for ( int d = 0; d < 3; ++d )
+    {
+        const int n = owned_hi( m, d ) - m.halo;
+        int head = 0, tail = 0;
+        if ( m.periodic[d] )
+        {
+            head = w + 1 - m.stag[d] < n ? w + 1 - m.stag[d] : n;
+            tail = w < n - head ? w : n - head;
+        }
+        s.d[d] = { m.halo, n, head, tail };
+    }
+    return s;
+}
+
+HaloGrids halo_grids( const GFieldDev* g, int ng )
+{
+    HaloGrids h = {};
+    for ( int i = 0; i < ng; ++i )
+        h.g[i] = g[i];
+    return h;
+}
+
+hipError_t launch_fill( Launcher& L, const char* name, bool fp64, const MeshDev& m,
+                        const GFieldDev* g, int ng, int width, int zero_other, int owners,
+                        hipStream_t s )
+{
+    const Shell shell = ghost_shell( m, g[0] );
+    const int64_t n = shell.size();
+    if ( n <= 0 )
+        return hipSuccess;
+    for ( int i = 0; i < ng; i += HALO_GRIDS )
+    {
+        const int k = ng - i < HALO_GRIDS ? ng - i : HALO_GRIDS;
+        dim3 grid = blocks_for( n );
+        grid.y = (unsigned)k;
+        L.before( name, s );
+        if ( fp64 )
+            hipLaunchKernelGGL( halo_fill_kernel<double>, grid, dim3( BLOCK ), 0, s, m,
+                                halo_grids( g + i, k ), shell, width, zero_other, owners );
+        else
+            hipLaunchKernelGGL( halo_fill_kernel<float>, grid, dim3( BLOCK ), 0, s, m,
+                                halo_grids( g + i, k ), shell, width, zero_other, owners );
+        L.after( name, s );
+    }
+    return hipGetLastError();
+}
+} // namespace
+
+hipError_t launch_halo_gather( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                               int ng, int width, hipStream_t s )
+{
+    return launch_fill( L, "halo_gather", fp64, m, g, ng, width, 0, 1, s );
+}
+
+hipError_t launch_halo_adjoint_fill( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                                     int ng, int width, hipStream_t s )
+{
+    return launch_fill( L, "halo_adjoint_fill", fp64, m, g, ng, width, 1, 1, s );
+}
+
+hipError_t launch_zero_ghosts( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                               int ng, hipStream_t s )
+{
+    return launch_fill( L, "zero_ghosts", fp64, m, g, ng, 0, 1, 0, s );
+}
+
+hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                                    int ng, int width, hipStream_t s )
+{
+    const Shell shell = image_shell( m, width );
+    const int64_t n = shell.size();
+    if ( n <= 0 )
+        return hipSuccess;
+    for ( int i = 0; i < ng; i += HALO_GRIDS )
+    {
+        const int k = ng - i < HALO_GRIDS ? ng - i : HALO_GRIDS;
+        dim3 grid = blocks_for( n );
+        grid.y = (unsigned)k;
+        L.before( "halo_scatter_sum", s );
+        if ( fp64 )
+            hipLaunchKernelGGL( halo_fold_kernel<double>, grid, dim3( BLOCK ), 0, s, m,
+                                halo_grids( g + i, k ), shell, width );
+        else
+            hipLaunchKernelGGL( halo_fold_kernel<float>, grid, dim3( BLOCK ), 0, s, m,
+                                halo_grids( g + i, k ), shell, width );
+        L.after( "halo_scatter_sum", s );
+    }
     return hipGetLastError();
 }
 
@@ -911,18 +1203,59 @@ int lcl_sort_passes( int key_bits, int* digit_bits )
     return passes;
 }
 
+hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out, int64_t n,
+                                  int64_t* block_sums, int64_t nblock_cap, hipStream_t s );
+
+namespace
+{
+hipError_t launch_lcl_bounds( Launcher& L, const int32_t* sorted_keys,
+                              int64_t n, int64_t ncell, int32_t* counts,
+                              int64_t* offsets, hipStream_t s )
+{
+    if ( ncell <= 0 )
+        return hipSuccess;
+    L.before( "lcl_bounds", s );
+    hipLaunchKernelGGL( lcl_bounds_kernel, blocks_for( ncell ), dim3( BLOCK ),
+                        0, s, sorted_keys, n, ncell, counts, offsets );
+    L.after( "lcl_bounds", s );
+    return hipGetLastError();
+}
+} // namespace
+
 hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
                             int32_t* keys_a, int32_t* keys_b, int32_t* vals_a,
                             int32_t* vals_b, int32_t* hist, int64_t* digit_base,
                             int64_t* block_sums, int64_t nblock_cap,
-                            int64_t* permutes, int64_t begin, int32_t** sorted,
-                            hipStream_t s )
+                            int64_t* permutes, int64_t begin, int64_t ncell,
+                            int32_t* counts, int64_t* offsets, hipStream_t s )
 {
-    *sorted = keys_a;
     if ( n <= 0 )
-        return hipSuccess;
+        return launch_lcl_bounds( L, keys_a, n, ncell, counts, offsets, s );
     int dbits;
     const int passes = lcl_sort_passes( key_bits, &dbits );
+    if ( n <= RS_SMALL_MAX )
+    {
+        // One workgroup (four or sixteen keys a thread).
+        const bool four = n <= 4 * RS_SMALL_BLOCK;
+        const size_t lds = four ? rs_small_lds<4>() : rs_small_lds<16>();
+        if ( lds > 64 * 1024 )
+        {
+            const hipError_t e = hipFuncSetAttribute(
+                reinterpret_cast<const void*>( lcl_sort_small_kernel<16> ),
+                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds );
+            if ( e != hipSuccess )
+                return e;
+        }
+        L.before( "lcl_sort_small", s );
+        hipLaunchKernelGGL( four ? lcl_sort_small_kernel<4> : lcl_sort_small_kernel<16>, dim3( 1 ),
+                            dim3( RS_SMALL_BLOCK ), lds, s, keys_a, (int)n, passes, dbits, permutes,
+                            begin, keys_b, ncell, counts, offsets );
+        L.after( "lcl_sort_small", s );
+        const hipError_t e = hipGetLastError();
+        if ( e != hipSuccess || ncell <= RS_SMALL_CELLS )
+            return e;
+        return launch_lcl_bounds( L, keys_b, n, ncell, counts, offsets, s );
+    }
     const int nbins = 1 << dbits;
     const int64_t ntiles = lcl_sort_tiles( n );
     int32_t* kin = keys_a;
@@ -975,21 +1308,7 @@ hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
         vin = vout;
         vout = t;
     }
-    *sorted = kin;
-    return hipSuccess;
-}
-
-hipError_t launch_lcl_bounds( Launcher& L, const int32_t* sorted_keys,
-                              int64_t n, int64_t ncell, int32_t* counts,
-                              int64_t* offsets, hipStream_t s )
-{
-    if ( ncell <= 0 )
-        return hipSuccess;
-    L.before( "lcl_bounds", s );
-    hipLaunchKernelGGL( lcl_bounds_kernel, blocks_for( ncell ), dim3( BLOCK ),
-                        0, s, sorted_keys, n, ncell, counts, offsets );
-    L.after( "lcl_bounds", s );
-    return hipGetLastError();
+    return launch_lcl_bounds( L, kin, n, ncell, counts, offsets, s );
 }
 
 hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
@@ -1002,6 +1321,12 @@ hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
     if ( nb > nblock_cap )
         return hipErrorInvalidValue;
     L.before( "exclusive_scan", s );
+    if ( n <= SCAN_ONE )
+    {
+        hipLaunchKernelGGL( scan_one_kernel, dim3( 1 ), dim3( SCAN_BLOCK ), 0, s, in, out, n );
+        L.after( "exclusive_scan", s );
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL( scan_reduce_kernel, dim3( (unsigned)nb ),
                         dim3( SCAN_BLOCK ), 0, s, in, n, block_sums );
     hipLaunchKernelGGL( scan_block_sums_kernel, dim3( 1 ), dim3( SCAN_BLOCK ),
@@ -1223,9 +1548,15 @@ hipError_t launch_brick_parts( Launcher& L, const TileArgs& t,
     if ( nbricks <= 0 )
         return hipErrorInvalidValue;
     L.before( "brick_parts", s );
-    hipLaunchKernelGGL( brick_count_kernel, blocks_for( nbricks ), dim3( BLOCK ), 0, s,
-                        t, make_int3( num_cell[0], num_cell[1], num_cell[2] ),
-                        brick_nparts );
+    hipLaunchKernelGGL( brick_count_kernel, blocks_for( nbricks * BRICK_LANES ), dim3( BLOCK ), 0,
+                        s, t, make_int3( num_cell[0], num_cell[1], num_cell[2] ), brick_nparts );
+    if ( nbricks <= SCAN_ONE )
+    {
+        hipLaunchKernelGGL( part_scan_fill_kernel, dim3( 1 ), dim3( SCAN_BLOCK ), 0, s,
+                            brick_nparts, (int)nbricks, parts, num_parts );
+        L.after( "brick_parts", s );
+        return hipGetLastError();
+    }
     L.after( "brick_parts", s );
     hipError_t e = launch_exclusive_scan( L, brick_nparts, brick_start, nbricks,
                                           block_sums, nblock_cap, s );

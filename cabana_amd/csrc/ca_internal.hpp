@@ -454,20 +454,19 @@ CABANA_AMD_DECLARE_LAUNCHERS( o4 )
 CABANA_AMD_DECLARE_LAUNCHERS( o5 )
 CABANA_AMD_DECLARE_LAUNCHERS( o6 )
 
-// Halo kernels on a ghosted node grid.
-hipError_t launch_halo_gather( Launcher& L, bool fp64, const MeshDev& m,
-                               const GFieldDev& g, int width, hipStream_t s );
-hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m,
-                                    const GFieldDev& g, int width,
-                                    hipStream_t s );
+// Halo kernels on ghosted arrays of one entity (ng arrays that share no
+// memory, in one launch).
+hipError_t launch_halo_gather( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                               int ng, int width, hipStream_t s );
+hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                                    int ng, int width, hipStream_t s );
 // Transpose of the fold for a cotangent grid: ghost := owner within the band,
 // 0 for every other non-owned node.
-hipError_t launch_halo_adjoint_fill( Launcher& L, bool fp64, const MeshDev& m,
-                                     const GFieldDev& g, int width,
-                                     hipStream_t s );
+hipError_t launch_halo_adjoint_fill( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                                     int ng, int width, hipStream_t s );
 // Zero every non-owned node.
-hipError_t launch_zero_ghosts( Launcher& L, bool fp64, const MeshDev& m,
-                               const GFieldDev& g, hipStream_t s );
+hipError_t launch_zero_ghosts( Launcher& L, bool fp64, const MeshDev& m, const GFieldDev* g,
+                               int ng, hipStream_t s );
 
 // Binning.
 struct CartGridDev
@@ -485,22 +484,18 @@ hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
                                   int64_t n, int64_t* block_sums,
                                   int64_t nblock_cap, hipStream_t s );
 // Stable radix sort of n keys in keys_a (values: the indices 0..n-1), digit
-// passes over key_bits bits.  Every pass needs hist (int32) and digit_base
-// (int64) of lcl_sort_bins * lcl_sort_tiles entries.  The sorted values
-// leave as begin + index in permutes; *sorted names the buffer holding the
-// sorted keys (keys_a or keys_b).
+// passes over key_bits bits, then counts[c] and offsets[c] of bins
+// 0..ncell-1.  Every pass needs hist (int32) and digit_base (int64) of
+// lcl_sort_bins * lcl_sort_tiles entries.  The sorted values leave as begin +
+// index in permutes.
 int64_t lcl_sort_tiles( int64_t n );
 int lcl_sort_passes( int key_bits, int* digit_bits );
 hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
                             int32_t* keys_a, int32_t* keys_b, int32_t* vals_a,
                             int32_t* vals_b, int32_t* hist, int64_t* digit_base,
                             int64_t* block_sums, int64_t nblock_cap,
-                            int64_t* permutes, int64_t begin, int32_t** sorted,
-                            hipStream_t s );
-// counts[c] and offsets[c] of bins 0..ncell-1 from n sorted keys.
-hipError_t launch_lcl_bounds( Launcher& L, const int32_t* sorted_keys,
-                              int64_t n, int64_t ncell, int32_t* counts,
-                              int64_t* offsets, hipStream_t s );
+                            int64_t* permutes, int64_t begin, int64_t ncell,
+                            int32_t* counts, int64_t* offsets, hipStream_t s );
 // Row-contiguous members of one particle set, permuted in one fused pass:
 // member f's rows are row_words[f] 4-byte words apart, words[f] of them per
 // particle, and its block of the scratch starts at n * word_offset[f] words.
