@@ -1198,7 +1198,8 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     int digit_bits;
     lcl_sort_passes( key_bits, &digit_bits );
     const int64_t nhist = ( (int64_t)1 << digit_bits ) * lcl_sort_tiles( n );
-    const int64_t nblock = ( nhist + 1023 ) / 1024 + 1;
+    const int64_t nscan = nhist > ncell ? nhist : ncell;
+    const int64_t nblock = ( nscan + 1023 ) / 1024 + 1;
     const int64_t nkey = n + 64;
     CA_HIP( ctx, ctx->ensure( SLOT_CELL_OF, sizeof( int32_t ) * 4 * nkey ), "scratch" );
     CA_HIP( ctx,
@@ -1216,12 +1217,22 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     int64_t* digit_base = static_cast<int64_t*>( ctx->scratch[SLOT_CURSOR] );
     int32_t* hist = reinterpret_cast<int32_t*>( digit_base + nhist + 64 );
     int64_t* sums = static_cast<int64_t*>( ctx->scratch[SLOT_SCAN] );
-    CA_HIP( ctx, launch_auto_bin_keys( *ctx, pts, n, m, keys, s ), "bin keys" );
-    CA_HIP( ctx,
-            launch_lcl_sort( *ctx, n, key_bits, keys, keys + nkey, keys + 2 * nkey,
-                             keys + 3 * nkey, hist, digit_base, sums, nblock, perm, 0, ncell,
-                             counts, offsets, s ),
-            "bin sort" );
+    if ( !ctx->deterministic && auto_bin_counts( n, ncell ) )
+    {
+        CA_HIP( ctx,
+                launch_auto_bin_count( *ctx, pts, n, m, ncell, keys, keys + nkey, counts, offsets,
+                                       sums, nblock, perm, s ),
+                "bin count" );
+    }
+    else
+    {
+        CA_HIP( ctx, launch_auto_bin_keys( *ctx, pts, n, m, keys, s ), "bin keys" );
+        CA_HIP( ctx,
+                launch_lcl_sort( *ctx, n, key_bits, keys, keys + nkey, keys + 2 * nkey,
+                                 keys + 3 * nkey, hist, digit_base, sums, nblock, perm, 0, ncell,
+                                 counts, offsets, s ),
+                "bin sort" );
+    }
     ctx->auto_bins = {};
     ctx->auto_bins.counts = counts;
     ctx->auto_bins.offsets = offsets;

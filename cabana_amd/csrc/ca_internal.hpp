@@ -554,6 +554,17 @@ hipError_t launch_migrate_shift( Launcher& L, const PFieldDev& pos, int64_t n,
 // (clamped into the owned cells).
 hipError_t launch_auto_bin_keys( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
                                  int32_t* keys, hipStream_t s );
+// The library's own binning by counting: cells counted with atomics as the
+// keys are formed, offsets by a scan, particles placed by their arrival
+// number.  Not stable (the order inside a cell varies), so the deterministic
+// mode sorts instead.
+hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
+                                  int64_t ncell, int32_t* keys, int32_t* rank, int32_t* counts,
+                                  int64_t* offsets, int64_t* block_sums, int64_t nblock_cap,
+                                  int64_t* perm, hipStream_t s );
+// Whether counting is used: beyond the one-workgroup sort, and where the cells
+// are not so few that their counters would be contended.
+bool auto_bin_counts( int64_t n, int64_t ncell );
 // Block [lo, lo + n) of every dimension of a grid array, packed x fastest
 // after the dofs (the BOV data order) into out.
 hipError_t launch_bov_pack( Launcher& L, bool fp64, const GFieldDev& g, int lo, const int n[3],
