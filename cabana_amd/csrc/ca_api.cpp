@@ -1226,11 +1226,10 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     }
     else
     {
-        CA_HIP( ctx, launch_auto_bin_keys( *ctx, pts, n, m, keys, s ), "bin keys" );
+        const SortScratch w = { keys, keys + nkey, keys + 2 * nkey, keys + 3 * nkey,
+                                hist, digit_base, sums, nblock };
         CA_HIP( ctx,
-                launch_lcl_sort( *ctx, n, key_bits, keys, keys + nkey, keys + 2 * nkey,
-                                 keys + 3 * nkey, hist, digit_base, sums, nblock, perm, 0, ncell,
-                                 counts, offsets, s ),
+                launch_auto_bin_sort( *ctx, pts, n, m, key_bits, w, perm, ncell, counts, offsets, s ),
                 "bin sort" );
     }
     ctx->auto_bins = {};
@@ -2346,14 +2345,11 @@ extern "C" cabana_amd_status cabana_amd_linked_cell_build(
             launch_fill_i32( *ctx, reinterpret_cast<int32_t*>( ctx->bad ), 2, 0,
                              s ),
             "fill" );
+    const SortScratch w = { keys, keys + nkey, keys + 2 * nkey, keys + 3 * nkey,
+                            hist, digit_base, sums, nblock };
     CA_HIP( ctx,
-            launch_lcl_keys( *ctx, pos, begin, end, g, (int32_t)ncell, keys,
-                             ctx->bad, s ),
-            "bin keys" );
-    CA_HIP( ctx,
-            launch_lcl_sort( *ctx, np, key_bits, keys, keys + nkey,
-                             keys + 2 * nkey, keys + 3 * nkey, hist, digit_base,
-                             sums, nblock, permutes, begin, ncell, counts, offsets, s ),
+            launch_lcl_build( *ctx, pos, begin, np, g, (int32_t)ncell, ctx->bad, key_bits, w,
+                              permutes, ncell, counts, offsets, s ),
             "bin sort" );
     // The reference fences after each phase; one wait here reports
     // particles outside the grid.

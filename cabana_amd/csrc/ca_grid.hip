@@ -115,11 +115,12 @@ __global__ __launch_bounds__( BLOCK ) void halo_fill_kernel( MeshDev m, HaloGrid
                                                              int w, int zero_other, int owners )
 {
     const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( e >= shell.size() )
-        return;
     const GFieldDev& g = gs.g[blockIdx.y];
+    if ( e >= shell.size() * g.ext[3] )
+        return;
+    const int dof = (int)( (uint32_t)e % (uint32_t)g.ext[3] );
     int x[3], o[3];
-    shell.at( (int)e, x );
+    shell.at( (int)( (uint32_t)e / (uint32_t)g.ext[3] ), x );
     bool reached = owners != 0;
 #pragma unroll
     for ( int d = 0; d < 3; ++d )
@@ -128,17 +129,11 @@ __global__ __launch_bounds__( BLOCK ) void halo_fill_kernel( MeshDev m, HaloGrid
         o[d] = owner_of( m, d, x[d], w, ghost );
         reached = reached && o[d] >= 0;
     }
-    Real* dst = gptr<Real>( g, x[0] * g.s[0] + x[1] * g.s[1] + x[2] * g.s[2] );
-    if ( !reached )
-    {
-        if ( zero_other )
-            for ( int d = 0; d < g.ext[3]; ++d )
-                dst[d * g.s[3]] = Real( 0 );
-        return;
-    }
-    const Real* src = gptr<const Real>( g, o[0] * g.s[0] + o[1] * g.s[1] + o[2] * g.s[2] );
-    for ( int d = 0; d < g.ext[3]; ++d )
-        dst[d * g.s[3]] = src[d * g.s[3]];
+    Real* dst = gptr<Real>( g, x[0] * g.s[0] + x[1] * g.s[1] + x[2] * g.s[2] + dof * g.s[3] );
+    if ( reached )
+        *dst = *gptr<const Real>( g, o[0] * g.s[0] + o[1] * g.s[1] + o[2] * g.s[2] + dof * g.s[3] );
+    else if ( zero_other )
+        *dst = Real( 0 );
 }
 
 // Fold: every owned node adds all of its periodic ghost images.  Each owner
@@ -149,11 +144,12 @@ __global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m, HaloGrid
                                                              int w )
 {
     const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( e >= shell.size() )
-        return;
     const GFieldDev& g = gs.g[blockIdx.y];
+    if ( e >= shell.size() * g.ext[3] )
+        return;
+    const int dof = (int)( (uint32_t)e % (uint32_t)g.ext[3] );
     int x[3];
-    shell.at( (int)e, x );
+    shell.at( (int)( (uint32_t)e / (uint32_t)g.ext[3] ), x );
     int cand[3][3], nc[3];
 #pragma unroll
     for ( int d = 0; d < 3; ++d )
@@ -169,23 +165,39 @@ __global__ __launch_bounds__( BLOCK ) void halo_fold_kernel( MeshDev m, HaloGrid
                 cand[d][nc[d]++] = x[d] - N;
         }
     }
-    Real* dst = gptr<Real>( g, x[0] * g.s[0] +
-                x[1] * g.s[1] + x[2] * g.s[2] );
-    for ( int d = 0; d < g.ext[3]; ++d )
+    Real* dst = gptr<Real>( g, x[0] * g.s[0] + x[1] * g.s[1] + x[2] * g.s[2] + dof * g.s[3] );
+    Real acc = Real( 0 );
+    if ( nc[0] <= 2 && nc[1] <= 2 && nc[2] <= 2 )
     {
-        Real acc = Real( 0 );
+        // Up to seven images, read together and summed in the order of the
+        // general loop.
+        Real v[8];
+#pragma unroll
+        for ( int q = 1; q < 8; ++q )
+        {
+            const int a = q >> 2, b = ( q >> 1 ) & 1, c = q & 1;
+            if ( a < nc[0] && b < nc[1] && c < nc[2] )
+                v[q] = *gptr<const Real>( g, cand[0][a] * g.s[0] + cand[1][b] * g.s[1] +
+                                                 cand[2][c] * g.s[2] + dof * g.s[3] );
+        }
+#pragma unroll
+        for ( int q = 1; q < 8; ++q )
+        {
+            const int a = q >> 2, b = ( q >> 1 ) & 1, c = q & 1;
+            if ( a < nc[0] && b < nc[1] && c < nc[2] )
+                acc += v[q];
+        }
+    }
+    else
+    {
         for ( int a = 0; a < nc[0]; ++a )
             for ( int b = 0; b < nc[1]; ++b )
                 for ( int c = 0; c < nc[2]; ++c )
-                {
-                    if ( a == 0 && b == 0 && c == 0 )
-                        continue;
-                    acc += *gptr<const Real>(
-                        g, cand[0][a] * g.s[0] + cand[1][b] * g.s[1] +
-                               cand[2][c] * g.s[2] + d * g.s[3] );
-                }
-        dst[d * g.s[3]] += acc;
+                    if ( a + b + c > 0 )
+                        acc += *gptr<const Real>( g, cand[0][a] * g.s[0] + cand[1][b] * g.s[1] +
+                                                         cand[2][c] * g.s[2] + dof * g.s[3] );
     }
+    *dst += acc;
 }
 
 // ---------------------------------------------------------------------------
@@ -216,22 +228,60 @@ __device__ __forceinline__ int64_t locate_cell( const CartGridDev& g,
 // Bin key of every particle in [begin, end): its cardinal cell, or bad_key
 // (one past the last cell) when the particle lies outside the grid.  No
 // per-cell counters are touched here: the counts come out of the sort.
-__global__ __launch_bounds__( BLOCK ) void lcl_key_kernel(
-    PFieldDev pos, int64_t begin, int64_t end, CartGridDev g, int32_t bad_key,
-    int32_t* keys, unsigned long long* bad )
+struct CartKey
+{
+    PFieldDev pos;
+    CartGridDev g;
+    int32_t bad_key;
+    unsigned long long* bad;
+    // Called by the lanes of a wave that hold a particle.
+    __device__ int32_t operator()( int64_t p ) const
+    {
+        const uint32_t b = pos.base( p );
+        const double x[3] = { *pos.ptr<const double>( b, 0 ),
+                              *pos.ptr<const double>( b, 1 ),
+                              *pos.ptr<const double>( b, 2 ) };
+        const int64_t c = locate_cell( g, x );
+        const unsigned long long out = __ballot( c < 0 );
+        if ( out && (int)( threadIdx.x & 63 ) == __ffsll( (long long)out ) - 1 )
+            atomicAdd( bad, (unsigned long long)__popcll( out ) );
+        return c < 0 ? bad_key : (int32_t)c;
+    }
+};
+
+// Owned cell of a particle for the library's own binning: clamped into the
+// owned cells (a particle in the halo or outside the domain still gets a
+// cell; the tiled kernels interpolate a particle whose stencil leaves its
+// brick through global memory).  Key = cardinal cell index.
+__device__ __forceinline__ int owned_cell( const PFieldDev& pos, int64_t p, const MeshDev& m )
+{
+#pragma clang fp contract( off )
+    const uint32_t b = pos.base( p );
+    int c[3];
+#pragma unroll
+    for ( int d = 0; d < 3; ++d )
+    {
+        const double x = *pos.ptr<const double>( b, d );
+        const double f = floor( ( x - m.low[d] ) * m.rdx[d] ) - (double)m.halo;
+        c[d] = f >= 0.0 ? ( f < (double)m.num_cell[d] ? (int)f : m.num_cell[d] - 1 ) : 0;
+    }
+    return ( c[0] * m.num_cell[1] + c[1] ) * m.num_cell[2] + c[2];
+}
+struct OwnedKey
+{
+    PFieldDev pos;
+    MeshDev m;
+    __device__ int32_t operator()( int64_t p ) const { return owned_cell( pos, p, m ); }
+};
+
+// Keys of particles [begin, end).
+template <class Key>
+__global__ __launch_bounds__( BLOCK ) void bin_key_kernel( Key key, int64_t begin, int64_t end,
+                                                           int32_t* keys )
 {
     const int64_t p = begin + (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( p >= end )
-        return;
-    const uint32_t b = pos.base( p );
-    const double x[3] = { *pos.ptr<const double>( b, 0 ),
-                          *pos.ptr<const double>( b, 1 ),
-                          *pos.ptr<const double>( b, 2 ) };
-    const int64_t c = locate_cell( g, x );
-    keys[p - begin] = c < 0 ? bad_key : (int32_t)c;
-    const unsigned long long out = __ballot( c < 0 );
-    if ( out && (int)( threadIdx.x & 63 ) == __ffsll( (long long)out ) - 1 )
-        atomicAdd( bad, (unsigned long long)__popcll( out ) );
+    if ( p < end )
+        keys[p - begin] = key( p );
 }
 
 constexpr int SCAN_BLOCK = 1024;
@@ -627,7 +677,8 @@ __global__ __launch_bounds__( BLOCK ) void lcl_bounds_kernel(
     counts[c] = (int32_t)( lower[threadIdx.x + 1] - lower[threadIdx.x] );
 }
 
-// The whole sort of up to RS_SMALL_BLOCK * ITEMS keys by one workgroup: every
+// The whole build of up to RS_SMALL_BLOCK * ITEMS particles by one workgroup:
+// the keys are formed in registers; every
 // pass stays in LDS (keys, 16-bit indices, per-wave digit counts), with the
 // ranks of radix_scatter_kernel; then the permutation and, for up to
 // RS_SMALL_CELLS bins, counts and offsets by binary search of the keys in LDS.
@@ -646,9 +697,9 @@ constexpr size_t rs_small_lds()
            sizeof( uint32_t ) * RS_SMALL_WAVES * RS_MAX_BINS;
 }
 
-template <int ITEMS>
+template <int ITEMS, class Key>
 __global__ __launch_bounds__( RS_SMALL_BLOCK ) void lcl_sort_small_kernel(
-    const int32_t* keys, int n, int passes, int dbits, int64_t* permutes, int64_t begin,
+    Key form_key, int n, int passes, int dbits, int64_t* permutes, int64_t begin,
     int32_t* sorted, int64_t ncell, int32_t* counts, int64_t* offsets )
 {
     extern __shared__ __align__( 16 ) unsigned char smem[];
@@ -667,7 +718,9 @@ __global__ __launch_bounds__( RS_SMALL_BLOCK ) void lcl_sort_small_kernel(
     for ( int k = 0; k < ITEMS; ++k )
     {
         const int i = wbase + k * 64 + lane;
-        key[k] = i < n ? keys[i] : 0;
+        key[k] = 0;
+        if ( i < n )
+            key[k] = form_key( begin + i );
         val[k] = (uint16_t)i;
     }
     for ( int p = 0; p < passes; ++p )
@@ -900,15 +953,11 @@ __global__ __launch_bounds__( BLOCK ) void permute_put_words_kernel(
 // parts of at most t.cap particles (an empty brick has none).
 // BRICK_LANES lanes sum the cell rows of a brick.
 constexpr int BRICK_LANES = 8;
-__global__ __launch_bounds__( BLOCK ) void brick_count_kernel( TileArgs t, int3 nc,
-                                                               int32_t* nparts )
+// Particles of brick b, to every lane of its group of BRICK_LANES.
+__device__ __forceinline__ int64_t brick_count( const TileArgs& t, int3 nc, int b, int sub )
 {
-    const int nbricks = t.ntile[0] * t.ntile[1] * t.ntile[2];
-    const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    const int b = (int)( e / BRICK_LANES );
-    const int sub = (int)( e % BRICK_LANES );
     int64_t count = 0;
-    if ( b < nbricks )
+    if ( b < t.ntile[0] * t.ntile[1] * t.ntile[2] )
     {
         const int bi = b / ( t.ntile[1] * t.ntile[2] );
         const int bj = ( b / t.ntile[2] ) % t.ntile[1];
@@ -928,8 +977,43 @@ __global__ __launch_bounds__( BLOCK ) void brick_count_kernel( TileArgs t, int3 
 #pragma unroll
     for ( int o = BRICK_LANES / 2; o > 0; o >>= 1 )
         count += __shfl_xor( count, o, 64 );
-    if ( b < nbricks && sub == 0 )
+    return count;
+}
+
+__global__ __launch_bounds__( BLOCK ) void brick_count_kernel( TileArgs t, int3 nc,
+                                                               int32_t* nparts )
+{
+    const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    const int b = (int)( e / BRICK_LANES );
+    const int64_t count = brick_count( t, nc, b, (int)( e % BRICK_LANES ) );
+    if ( b < t.ntile[0] * t.ntile[1] * t.ntile[2] && e % BRICK_LANES == 0 )
         nparts[b] = (int32_t)( ( count + t.cap - 1 ) / t.cap );
+}
+
+// The whole part table of a small mesh in one launch: up to PART_SMALL cell
+// rows in all, BRICK_LANES lanes a brick, counts in LDS (256 rows: 6 us against
+// 10 us for two launches; 8192 rows: 15 us, the reads of one workgroup).
+constexpr int PART_SMALL = 2048;
+constexpr int PART_SMALL_BRICKS = 2048;
+__global__ __launch_bounds__( SCAN_BLOCK ) void part_small_kernel( TileArgs t, int3 nc,
+                                                                   int2* parts, int32_t* num_parts )
+{
+    __shared__ int32_t nparts[PART_SMALL_BRICKS];
+    const int nbricks = t.ntile[0] * t.ntile[1] * t.ntile[2];
+    for ( int b0 = 0; b0 < nbricks; b0 += SCAN_BLOCK / BRICK_LANES )
+    {
+        const int b = b0 + (int)threadIdx.x / BRICK_LANES;
+        const int64_t count = brick_count( t, nc, b, threadIdx.x % BRICK_LANES );
+        if ( b < nbricks && threadIdx.x % BRICK_LANES == 0 )
+            nparts[b] = (int32_t)( ( count + t.cap - 1 ) / t.cap );
+    }
+    __syncthreads();
+    const int64_t total = scan_one( nparts, nbricks, [&]( int b, int32_t np, int64_t before ) {
+        for ( int q = 0; q < np; ++q )
+            parts[before + q] = make_int2( b, q );
+    } );
+    if ( threadIdx.x == 0 )
+        *num_parts = (int32_t)total;
 }
 
 // Scan of the bricks' part counts and the part table in one launch (up to
@@ -1052,34 +1136,6 @@ __global__ __launch_bounds__( BLOCK ) void compact_index_kernel( const int32_t* 
         idx[rank[p]] = p;
 }
 
-// Cell of a particle for the library's own binning of a call that passes
-// none: the floor of its logical cell coordinate in the owned cells,
-// clamped into them (a particle outside them, or with a NaN coordinate,
-// still gets a cell; the tiled kernels interpolate a particle whose stencil
-// leaves its brick through global memory).  Key = cardinal cell index.
-__device__ __forceinline__ int owned_cell( const PFieldDev& pos, int64_t p, const MeshDev& m )
-{
-#pragma clang fp contract( off )
-    const uint32_t b = pos.base( p );
-    int c[3];
-#pragma unroll
-    for ( int d = 0; d < 3; ++d )
-    {
-        const double x = *pos.ptr<const double>( b, d );
-        const double f = floor( ( x - m.low[d] ) * m.rdx[d] ) - (double)m.halo;
-        c[d] = f >= 0.0 ? ( f < (double)m.num_cell[d] ? (int)f : m.num_cell[d] - 1 ) : 0;
-    }
-    return ( c[0] * m.num_cell[1] + c[1] ) * m.num_cell[2] + c[2];
-}
-
-__global__ __launch_bounds__( BLOCK ) void auto_bin_key_kernel( PFieldDev pos, int64_t n,
-                                                                MeshDev m, int32_t* keys )
-{
-    const int64_t p = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( p < n )
-        keys[p] = owned_cell( pos, p, m );
-}
-
 // The same keys counted as they are formed: rank[p] is the particle's arrival
 // number in its cell.  Lanes of a wave with equal keys next to each other
 // (particles near cell order) share one atomic.
@@ -1188,6 +1244,15 @@ HaloGrids halo_grids( const GFieldDev* g, int ng )
     return h;
 }
 
+// Dofs of the widest of ng grids (a thread per node and dof).
+int most_dofs( const GFieldDev* g, int ng )
+{
+    int n = 1;
+    for ( int i = 0; i < ng; ++i )
+        n = g[i].ext[3] > n ? g[i].ext[3] : n;
+    return n;
+}
+
 hipError_t launch_fill( Launcher& L, const char* name, bool fp64, const MeshDev& m,
                         const GFieldDev* g, int ng, int width, int zero_other, int owners,
                         hipStream_t s )
@@ -1199,7 +1264,7 @@ hipError_t launch_fill( Launcher& L, const char* name, bool fp64, const MeshDev&
     for ( int i = 0; i < ng; i += HALO_GRIDS )
     {
         const int k = ng - i < HALO_GRIDS ? ng - i : HALO_GRIDS;
-        dim3 grid = blocks_for( n );
+        dim3 grid = blocks_for( n * most_dofs( g + i, k ) );
         grid.y = (unsigned)k;
         L.before( name, s );
         if ( fp64 )
@@ -1242,7 +1307,7 @@ hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m, co
     for ( int i = 0; i < ng; i += HALO_GRIDS )
     {
         const int k = ng - i < HALO_GRIDS ? ng - i : HALO_GRIDS;
-        dim3 grid = blocks_for( n );
+        dim3 grid = blocks_for( n * most_dofs( g + i, k ) );
         grid.y = (unsigned)k;
         L.before( "halo_scatter_sum", s );
         if ( fp64 )
@@ -1253,21 +1318,6 @@ hipError_t launch_halo_scatter_sum( Launcher& L, bool fp64, const MeshDev& m, co
                                 halo_grids( g + i, k ), shell, width );
         L.after( "halo_scatter_sum", s );
     }
-    return hipGetLastError();
-}
-
-hipError_t launch_lcl_keys( Launcher& L, const PFieldDev& pos, int64_t begin,
-                            int64_t end, const CartGridDev& g, int32_t bad_key,
-                            int32_t* keys, unsigned long long* bad,
-                            hipStream_t s )
-{
-    if ( end <= begin )
-        return hipSuccess;
-    L.before( "lcl_keys", s );
-    hipLaunchKernelGGL( lcl_key_kernel, blocks_for( end - begin ),
-                        dim3( BLOCK ), 0, s, pos, begin, end, g, bad_key, keys,
-                        bad );
-    L.after( "lcl_keys", s );
     return hipGetLastError();
 }
 
@@ -1302,46 +1352,64 @@ hipError_t launch_lcl_bounds( Launcher& L, const int32_t* sorted_keys,
 }
 } // namespace
 
-hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
-                            int32_t* keys_a, int32_t* keys_b, int32_t* vals_a,
-                            int32_t* vals_b, int32_t* hist, int64_t* digit_base,
-                            int64_t* block_sums, int64_t nblock_cap,
-                            int64_t* permutes, int64_t begin, int64_t ncell,
-                            int32_t* counts, int64_t* offsets, hipStream_t s )
+namespace
+{
+template <int ITEMS, class Key>
+hipError_t launch_sort_small( Launcher& L, const char* name, const Key& key, int64_t begin, int64_t n, int passes,
+                              int dbits, int64_t* permutes, int32_t* sorted, int64_t ncell,
+                              int32_t* counts, int64_t* offsets, hipStream_t s )
+{
+    constexpr size_t lds = rs_small_lds<ITEMS>();
+    if ( lds > 64 * 1024 )
+    {
+        const hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void*>( lcl_sort_small_kernel<ITEMS, Key> ),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds );
+        if ( e != hipSuccess )
+            return e;
+    }
+    L.before( name, s );
+    hipLaunchKernelGGL( ( lcl_sort_small_kernel<ITEMS, Key> ), dim3( 1 ), dim3( RS_SMALL_BLOCK ),
+                        lds, s, key, (int)n, passes, dbits, permutes, begin, sorted, ncell, counts,
+                        offsets );
+    L.after( name, s );
+    return hipGetLastError();
+}
+
+template <class Key>
+hipError_t bin_sort( Launcher& L, const char* name, const Key& key, int64_t begin, int64_t n, int key_bits,
+                     const SortScratch& w, int64_t* permutes, int64_t ncell, int32_t* counts,
+                     int64_t* offsets, hipStream_t s )
 {
     if ( n <= 0 )
-        return launch_lcl_bounds( L, keys_a, n, ncell, counts, offsets, s );
+        return launch_lcl_bounds( L, w.keys_a, n, ncell, counts, offsets, s );
     int dbits;
     const int passes = lcl_sort_passes( key_bits, &dbits );
     if ( n <= RS_SMALL_MAX )
     {
         // One workgroup (four or sixteen keys a thread).
-        const bool four = n <= 4 * RS_SMALL_BLOCK;
-        const size_t lds = four ? rs_small_lds<4>() : rs_small_lds<16>();
-        if ( lds > 64 * 1024 )
-        {
-            const hipError_t e = hipFuncSetAttribute(
-                reinterpret_cast<const void*>( lcl_sort_small_kernel<16> ),
-                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds );
-            if ( e != hipSuccess )
-                return e;
-        }
-        L.before( "lcl_sort_small", s );
-        hipLaunchKernelGGL( four ? lcl_sort_small_kernel<4> : lcl_sort_small_kernel<16>, dim3( 1 ),
-                            dim3( RS_SMALL_BLOCK ), lds, s, keys_a, (int)n, passes, dbits, permutes,
-                            begin, keys_b, ncell, counts, offsets );
-        L.after( "lcl_sort_small", s );
-        const hipError_t e = hipGetLastError();
+        const hipError_t e =
+            n <= 4 * RS_SMALL_BLOCK
+                ? launch_sort_small<4>( L, name, key, begin, n, passes, dbits, permutes, w.keys_b, ncell,
+                                        counts, offsets, s )
+                : launch_sort_small<16>( L, name, key, begin, n, passes, dbits, permutes, w.keys_b, ncell,
+                                         counts, offsets, s );
         if ( e != hipSuccess || ncell <= RS_SMALL_CELLS )
             return e;
-        return launch_lcl_bounds( L, keys_b, n, ncell, counts, offsets, s );
+        return launch_lcl_bounds( L, w.keys_b, n, ncell, counts, offsets, s );
     }
+    L.before( name, s );
+    hipLaunchKernelGGL( bin_key_kernel<Key>, blocks_for( n ), dim3( BLOCK ), 0, s, key, begin,
+                        begin + n, w.keys_a );
+    L.after( name, s );
+    int32_t* hist = w.hist;
+    int64_t* digit_base = w.digit_base;
     const int nbins = 1 << dbits;
     const int64_t ntiles = lcl_sort_tiles( n );
-    int32_t* kin = keys_a;
-    int32_t* kout = keys_b;
-    int32_t* vin = vals_a;
-    int32_t* vout = vals_b;
+    int32_t* kin = w.keys_a;
+    int32_t* kout = w.keys_b;
+    int32_t* vin = w.vals_a;
+    int32_t* vout = w.vals_b;
     for ( int p = 0; p < passes; ++p )
     {
         const int shift = p * dbits;
@@ -1352,7 +1420,7 @@ hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
         L.after( "lcl_sort_hist", s );
         hipError_t e = launch_exclusive_scan( L, hist, digit_base,
                                               (int64_t)nbins * ntiles,
-                                              block_sums, nblock_cap, s );
+                                              w.block_sums, w.nblock_cap, s );
         if ( e != hipSuccess )
             return e;
         const bool first = p == 0, last = p == passes - 1;
@@ -1389,6 +1457,24 @@ hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
         vout = t;
     }
     return launch_lcl_bounds( L, kin, n, ncell, counts, offsets, s );
+}
+} // namespace
+
+hipError_t launch_lcl_build( Launcher& L, const PFieldDev& pos, int64_t begin, int64_t n,
+                             const CartGridDev& g, int32_t bad_key, unsigned long long* bad,
+                             int key_bits, const SortScratch& w, int64_t* permutes, int64_t ncell,
+                             int32_t* counts, int64_t* offsets, hipStream_t s )
+{
+    return bin_sort( L, "lcl_keys", CartKey{ pos, g, bad_key, bad }, begin, n, key_bits, w, permutes, ncell,
+                     counts, offsets, s );
+}
+
+hipError_t launch_auto_bin_sort( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
+                                 int key_bits, const SortScratch& w, int64_t* permutes,
+                                 int64_t ncell, int32_t* counts, int64_t* offsets, hipStream_t s )
+{
+    return bin_sort( L, "auto_bin_keys", OwnedKey{ pos, m }, 0, n, key_bits, w, permutes, ncell,
+                     counts, offsets, s );
 }
 
 hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
@@ -1628,6 +1714,13 @@ hipError_t launch_brick_parts( Launcher& L, const TileArgs& t,
     if ( nbricks <= 0 )
         return hipErrorInvalidValue;
     L.before( "brick_parts", s );
+    if ( nbricks <= PART_SMALL_BRICKS && nbricks * t.tile[0] * t.tile[1] <= PART_SMALL )
+    {
+        hipLaunchKernelGGL( part_small_kernel, dim3( 1 ), dim3( SCAN_BLOCK ), 0, s, t,
+                            make_int3( num_cell[0], num_cell[1], num_cell[2] ), parts, num_parts );
+        L.after( "brick_parts", s );
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL( brick_count_kernel, blocks_for( nbricks * BRICK_LANES ), dim3( BLOCK ), 0,
                         s, t, make_int3( num_cell[0], num_cell[1], num_cell[2] ), brick_nparts );
     if ( nbricks <= SCAN_ONE )
@@ -1704,18 +1797,6 @@ hipError_t launch_bov_pack( Launcher& L, bool fp64, const GFieldDev& g, int lo, 
     return hipGetLastError();
 }
 
-hipError_t launch_auto_bin_keys( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
-                                 int32_t* keys, hipStream_t s )
-{
-    if ( n <= 0 )
-        return hipSuccess;
-    L.before( "auto_bin_keys", s );
-    hipLaunchKernelGGL( auto_bin_key_kernel, blocks_for( n ), dim3( BLOCK ), 0, s, pos, n, m,
-                        keys );
-    L.after( "auto_bin_keys", s );
-    return hipGetLastError();
-}
-
 hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
                                   int64_t ncell, int32_t* keys, int32_t* rank, int32_t* counts,
                                   int64_t* offsets, int64_t* block_sums, int64_t nblock_cap,
@@ -1724,10 +1805,10 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
     hipError_t e = launch_fill_i32( L, counts, ncell, 0, s );
     if ( e != hipSuccess )
         return e;
-    L.before( "auto_bin_rank", s );
+    L.before( "auto_bin_keys", s );
     hipLaunchKernelGGL( auto_bin_rank_kernel, blocks_for( n ), dim3( BLOCK ), 0, s, pos, n, m, keys,
                         counts, rank );
-    L.after( "auto_bin_rank", s );
+    L.after( "auto_bin_keys", s );
     e = launch_exclusive_scan( L, counts, offsets, ncell, block_sums, nblock_cap, s );
     if ( e != hipSuccess )
         return e;

@@ -475,27 +475,38 @@ struct CartGridDev
     double rdx[3];
     int32_t nx[3];
 };
-// Bin keys (cell index, or bad_key outside the grid) of [begin, end).
-hipError_t launch_lcl_keys( Launcher& L, const PFieldDev& pos, int64_t begin,
-                            int64_t end, const CartGridDev& g, int32_t bad_key,
-                            int32_t* keys, unsigned long long* bad,
-                            hipStream_t s );
 hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
                                   int64_t n, int64_t* block_sums,
                                   int64_t nblock_cap, hipStream_t s );
-// Stable radix sort of n keys in keys_a (values: the indices 0..n-1), digit
-// passes over key_bits bits, then counts[c] and offsets[c] of bins
-// 0..ncell-1.  Every pass needs hist (int32) and digit_base (int64) of
-// lcl_sort_bins * lcl_sort_tiles entries.  The sorted values leave as begin +
-// index in permutes.
+// Scratch of a sorting build of n particles: keys and values of two buffers
+// (n + 64 int32 each), hist (int32) and digit_base (int64) of 2^digit_bits *
+// lcl_sort_tiles( n ) + 64 entries, block sums of the scans.
+struct SortScratch
+{
+    int32_t* keys_a;
+    int32_t* keys_b;
+    int32_t* vals_a;
+    int32_t* vals_b;
+    int32_t* hist;
+    int64_t* digit_base;
+    int64_t* block_sums;
+    int64_t nblock_cap;
+};
 int64_t lcl_sort_tiles( int64_t n );
 int lcl_sort_passes( int key_bits, int* digit_bits );
-hipError_t launch_lcl_sort( Launcher& L, int64_t n, int key_bits,
-                            int32_t* keys_a, int32_t* keys_b, int32_t* vals_a,
-                            int32_t* vals_b, int32_t* hist, int64_t* digit_base,
-                            int64_t* block_sums, int64_t nblock_cap,
-                            int64_t* permutes, int64_t begin, int64_t ncell,
-                            int32_t* counts, int64_t* offsets, hipStream_t s );
+// Bins particles [begin, begin + n): keys (cell index, or bad_key outside the
+// grid, counted in *bad), a stable radix sort of them over key_bits bits,
+// counts[c] and offsets[c] of bins 0..ncell-1.  The sorted order leaves as
+// begin + index in permutes.
+hipError_t launch_lcl_build( Launcher& L, const PFieldDev& pos, int64_t begin, int64_t n,
+                             const CartGridDev& g, int32_t bad_key, unsigned long long* bad,
+                             int key_bits, const SortScratch& w, int64_t* permutes, int64_t ncell,
+                             int32_t* counts, int64_t* offsets, hipStream_t s );
+// The same with owned-cell keys (clamped into the owned cells) of particles
+// [0, n), for the library's own binning.
+hipError_t launch_auto_bin_sort( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
+                                 int key_bits, const SortScratch& w, int64_t* permutes,
+                                 int64_t ncell, int32_t* counts, int64_t* offsets, hipStream_t s );
 // Row-contiguous members of one particle set, permuted in one fused pass:
 // member f's rows are row_words[f] 4-byte words apart, words[f] of them per
 // particle, and its block of the scratch starts at n * word_offset[f] words.
@@ -550,10 +561,6 @@ hipError_t launch_migrate_count( Launcher& L, const PFieldDev& pos, int64_t n,
 hipError_t launch_migrate_shift( Launcher& L, const PFieldDev& pos, int64_t n,
                                  const MigrateBoundsDev& b, int32_t* keep,
                                  unsigned long long* dropped, hipStream_t s );
-// Owned-cell keys of particles [0, n) for the library's own binning
-// (clamped into the owned cells).
-hipError_t launch_auto_bin_keys( Launcher& L, const PFieldDev& pos, int64_t n, const MeshDev& m,
-                                 int32_t* keys, hipStream_t s );
 // The library's own binning by counting: cells counted with atomics as the
 // keys are formed, offsets by a scan, particles placed by their arrival
 // number.  Not stable (the order inside a cell varies), so the deterministic
