@@ -750,8 +750,8 @@ size_t tile_lds_bytes( TileKind kind, bool fp64, const int* slot_ng, int nslot, 
     for ( int i = 0; i < nslot; ++i )
         dt += slot_ng[i];
     b = a16( 8 * (size_t)dt * wn );
-    b = a16( b + real * ( SCATTER_BLOCK / 64 ) * ( scatter_sub( scatter_row( vals ) ) + 3 ) *
-                     scatter_record( fp64, scatter_row( vals ) ) );
+    b = a16( b + real * ( SCATTER_BLOCK / 64 ) * ( scatter_sub( scatter_grad( vals ) ) + 3 ) *
+                     scatter_record( fp64, order, scatter_row( order, vals ) ) );
     b = a16( b + 8 * runs );
     b = a16( b + 4 * ( runs + 1 ) );
     return b;
@@ -797,7 +797,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
     // the part table itself is large, two workgroups per CU.
     const int extra = ( order == 1 ) ? 1 : 3;
     const int c = scatter_cells_k( order );
-    const int waves = scatter_waves( fp64, scatter_row( vals ) );
+    const int waves = scatter_waves( fp64, scatter_grad( vals ) );
     bool found = false;
     double best_bricks = 0.0;
     for ( int w = waves; w >= 2 && ( !found || best_bricks > 1048576.0 ); w = w > 2 ? 2 : 1 )

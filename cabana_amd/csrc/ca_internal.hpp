@@ -364,17 +364,23 @@ struct TileArgs
     }
 };
 
-// Cell-tiled scatter (ca_scatter.hip).  A pass is of one of two kinds, by the
-// values in a slot of its records (scatter_row): four with value-type terms
-// only, six with gradient-type ones.
+// Cell-tiled scatter (ca_scatter.hip).  A pass is of one of two kinds: with
+// value-type terms only, or with gradient-type ones (`grad`: three more
+// values in a slot of its records).
 constexpr int SCATTER_BLOCK = 256;
-constexpr int scatter_row( int vals ) { return ( 2 + vals + 1 ) / 2 * 2; }
+constexpr bool scatter_grad( int vals ) { return vals >= 3; }
+// Weights at the head of a slot row, and the row with its values, even.
+constexpr int scatter_row_head( int order, bool grad ) { return order == 1 ? ( grad ? 3 : 1 ) : 2; }
+constexpr int scatter_row( int order, int vals )
+{
+    return ( scatter_row_head( order, scatter_grad( vals ) ) + vals + 1 ) / 2 * 2;
+}
 // Waves per SIMD the registers of a pass leave room for without spilling
 // (a spill of a few registers at one wave more measured 1.2 to 2 times
 // slower), and the LDS that lets as many workgroups run on a CU.
-constexpr int scatter_waves( bool fp64, int row )
+constexpr int scatter_waves( bool fp64, bool grad )
 {
-    return fp64 ? ( row == 4 ? 3 : 2 ) : ( row == 4 ? 4 : 3 );
+    return fp64 ? ( grad ? 2 : 3 ) : ( grad ? 3 : 4 );
 }
 constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
 // Particles of a wave's batch of 64 whose records are in LDS at a time.
@@ -382,16 +388,17 @@ constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
 // SIMD); 16 break more groups apart: at 128^3 x 16 FP32 the MPM P2G takes
 // 1.51 ms with 32 and 1.67 ms with 16, and mass and momentum of 8.4 M clustered
 // particles, whose windows are larger, 0.50 ms with 32 and 0.46 ms with 16.
-constexpr int scatter_sub( int row ) { return row == 4 ? 16 : 32; }
+constexpr int scatter_sub( bool grad ) { return grad ? 32 : 16; }
 // Cells of a scatter brick along k, a compile-time stride of the LDS window
 // (linear splines: groups of three cells).
 constexpr int scatter_cells_k( int order ) { return order == 1 ? 9 : 8; }
-// A scatter record: 16 weights and four slot rows of `row` values, with a
+// A scatter record: 16 weights (linear splines: 8) and four slot rows, with a
 // stride that puts the 16-byte pieces eight lanes write at a time into
 // different LDS banks.
-constexpr int scatter_record( bool fp64, int row )
+constexpr int scatter_record( bool fp64, int order, int row )
 {
-    return 16 + 4 * row + ( fp64 ? 2 : ( row == 4 ? 4 : 0 ) );
+    const int len = ( order == 1 ? 8 : 16 ) + 4 * row;
+    return len + ( fp64 ? 2 : ( len % 8 == 0 && len % 16 != 0 ? 0 : 4 ) );
 }
 
 // Launch-time error/timing context owned by the C-ABI layer.

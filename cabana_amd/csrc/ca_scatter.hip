@@ -14,6 +14,24 @@
 // walks its share of the part, 64 particles a batch (one per lane: positions,
 // weights and attributes, written to the wave's records in LDS), then the
 // batch's runs of equal cell, four particles a step.
+//
+// Linear splines reach 2 x 2 nodes along (i, j), four rows of the sixteen:
+// v_mfma_*_4x4x* takes the same four particles a step with rows (i, j) and
+// columns d, a block for every k (and, in FP32, every particle), at a quarter
+// of the matrix time.
+//
+// What bounds it: instruction issue.  FP32 matrix and vector instructions do
+// not overlap on a SIMD of this chip (137 and 166 cycles of each alone take 299
+// together), so a batch of 64 particles of the MPM P2G, quadratic, FP32, costs
+// the 2930 vector and 2340 matrix cycles of its wave one after the other, and
+// waits for LDS take most of the remaining 1700.  HBM moves 2.6 GB in 1.52 ms.
+// Against the kernel this one replaced, which sorted each task's particles in
+// LDS and added their 27 nodes by LDS atomics, spent half its time at barriers:
+//   MPM P2G, 33.6 M particles of 128^3 cells, quadratic, FP32  2.47 -> 1.52 ms
+//   MPM P2G, odd grid, cubic, FP64                             0.70 -> 0.36 ms
+//   mass and momentum, 8.4 M clustered particles, FP32         0.70 -> 0.46 ms
+//   MPM P2G, 7.1 M particles of 96^3 cells, linear, FP64       0.43 -> 0.39 ms
+// (linear splines in 16 x 16 products: 0.52 ms).
 #include "ca_tiles.hpp"
 
 namespace cabana_amd
@@ -57,11 +75,11 @@ struct Tiles
             r = r || !value_form( FL::v[t] );
         return r;
     }
-    // Offset of a tile's values in a record's slot row, after its weight and
-    // gradient.
+    static constexpr bool any_g() { return has_g( 0 ) || has_g( NT - 1 ); }
+    // Offset of a tile's values in a record's slot row, after its weights.
     static constexpr int val( int tile )
     {
-        int o = 2;
+        int o = scatter_row_head( ORDER, any_g() );
         for ( int i = 0; i < tile; ++i )
             o += ( has_v( i ) ? 1 : 0 ) + ( has_g( i ) ? 3 : 0 );
         return o;
@@ -80,16 +98,21 @@ struct Tiles
 // Record of a particle: weight and gradient along QUAD and along k of the four
 // window nodes, then the four slot rows (weight and gradient along SLOT of the
 // node with the slot's number, then the slot's values) in 16-byte chunks,
-// [chunk][slot].  The record stride spreads the four records of a step over
+// [chunk][slot].  Linear splines: weight and gradient along k of the four
+// window nodes, then slot rows that begin with the products of the x and y
+// weights of the (i, j) node with the slot's number (value, x and y gradient).
+// The record stride spreads the four records of a step over
 // the LDS banks.
 template <class Real, int ROW>
 struct Record
 {
+    // Values before the slot rows (linear splines: along k only).
+    static constexpr int HEAD = ORDER == 1 ? 8 : 16;
     static constexpr int CW = 16 / (int)sizeof( Real );
     static constexpr int NC = ( ROW + CW - 1 ) / CW;
-    static constexpr int STRIDE = scatter_record( sizeof( Real ) == 8, ROW );
+    static constexpr int STRIDE = scatter_record( sizeof( Real ) == 8, ORDER, ROW );
     static constexpr int width( int c ) { return ROW - c * CW < CW ? ROW - c * CW : CW; }
-    static constexpr int at( int c, int slot ) { return 16 + 4 * CW * c + slot * width( c ); }
+    static constexpr int at( int c, int slot ) { return HEAD + 4 * CW * c + slot * width( c ); }
     template <int N>
     struct Vec
     {
@@ -109,6 +132,12 @@ struct Record
     static __device__ __forceinline__ void put_pair( Real* at, Real w, Real g )
     {
         *reinterpret_cast<typename Vec<2>::type*>( at ) = typename Vec<2>::type{ w, g };
+    }
+    static __device__ __forceinline__ void get_pair( const Real* at, Real& w, Real& g )
+    {
+        const auto x = *reinterpret_cast<const typename Vec<2>::type*>( at );
+        w = x[0];
+        g = x[1];
     }
     static __device__ __forceinline__ void get_row( const Real* rec, int slot, Real* v )
     {
@@ -181,6 +210,27 @@ struct Mfma<double>
         return __builtin_amdgcn_mfma_f64_16x16x4f64( a, b, c, 0, 0, 0 );
     }
 };
+
+// Accumulators of a tile and a chunk's sums.  In the 4 x 4 products of linear
+// splines lane l holds column l % 4 of block l / 4: in FP32 rows r = (i, j) of
+// register r, a block for each particle of the step (l / 16) and each k; in
+// FP64 row l / 16 and a block for each k.
+template <class Real>
+constexpr int acc_regs()
+{
+    return ORDER == 1 && sizeof( Real ) == 8 ? 1 : 4;
+}
+[[maybe_unused]] __device__ __forceinline__ Mfma<float>::V4
+mac4( float a, float b, Mfma<float>::V4 c )
+{
+    return __builtin_amdgcn_mfma_f32_4x4x1f32( a, b, c, 0, 0, 0 );
+}
+[[maybe_unused]] __device__ __forceinline__ Mfma<double>::V4
+mac4( double a, double b, Mfma<double>::V4 c )
+{
+    c[0] = __builtin_amdgcn_mfma_f64_4x4x4f64( a, b, c[0], 0, 0, 0 );
+    return c;
+}
 
 // DPP move: lane Q of every quad to its four lanes.
 template <int CTRL>
@@ -383,12 +433,13 @@ constexpr int WK = scatter_cells_k( ORDER ) + ( ORDER == 1 ? 1 : 3 );
 template <class Real, int ROW>
 struct Step
 {
-    Real xz;
+    Real xz; // one weight of the quad's four (linear splines: wz)
+    Real gz; // linear splines
     Real y[ROW];
 };
 
 template <class Real, bool CONTIG, bool SHARED, int... FORMS>
-__global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 8, Tiles<SHARED, FORMS...>::row() ) ) ) void scatter_cells_kernel(
+__global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 8, Tiles<SHARED, FORMS...>::any_g() ) ) ) void scatter_cells_kernel(
     ScatterArgs a, TileArgs ta )
 {
     using FL = FormList<FORMS...>;
@@ -401,7 +452,8 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     constexpr int RS = RC::STRIDE;
     constexpr int NP = attr_len<FORMS...>();
     constexpr int NWAVE = SCATTER_BLOCK / 64;
-    constexpr int SUB = scatter_sub( ROW );
+    constexpr int SUB = scatter_sub( TL::any_g() );
+    constexpr int NR = acc_regs<Real>();
     constexpr bool F32 = sizeof( Real ) == 4;
     // Window nodes along k sit in column (node index mod 4), so that the
     // window slides to the next cell without moving the accumulators.  (The
@@ -471,19 +523,23 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
 
         // The open window: key of the group in the accumulators, -1 none.
         int open = -1;
-        double acc[NT][4];
+        double acc[NT][NR];
 #pragma unroll
         for ( int t = 0; t < NT; ++t )
 #pragma unroll
-            for ( int r = 0; r < 4; ++r )
+            for ( int r = 0; r < NR; ++r )
                 acc[t][r] = 0.0;
         // Adds the accumulators to the LDS window (all columns, or the window's
         // first node along k) and clears them.
         auto retire = [&]( int key, bool all ) {
             const int dk = SLIDE ? ( kcol - key ) & 3 : kcol;
-            const int node = ( ( ( key >> 16 ) + pslot ) * W[1] + ( ( key >> 8 ) & 255 ) ) * WK +
+            // Window node of accumulator register r: (i, j) = (lane / 16, r),
+            // or for linear splines r (FP32) or lane / 16 (FP64) = 2 i + j.
+            const int i0 = ORDER > 1 ? pslot : ( F32 ? 0 : pslot >> 1 );
+            const int j0 = ORDER > 1 || F32 ? 0 : pslot & 1;
+            const int node = ( ( ( key >> 16 ) + i0 ) * W[1] + ( ( key >> 8 ) & 255 ) + j0 ) * WK +
                              ( key & 255 ) + dk;
-            const bool on = ( all || dk == 0 ) && ( ORDER > 1 || pslot < 2 );
+            const bool on = all || dk == 0;
             int wo = 0;
             static_for<NT>( [&]( auto T ) {
                 constexpr int t = T;
@@ -492,8 +548,9 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                 {
                     double* q = win + ( wo + node * ND + slot );
 #pragma unroll
-                    for ( int r = 0; r < ( ORDER > 1 ? 4 : 2 ); ++r )
-                        atomicAdd( q + r * WK * ND, acc[t][r] );
+                    for ( int r = 0; r < NR; ++r )
+                        atomicAdd( q + ( ORDER > 1 ? r * WK : ( ( r >> 1 ) * W[1] + ( r & 1 ) ) * WK ) * ND,
+                                   acc[t][r] );
                 }
                 wo += ta.max_win_nodes * ND;
             } );
@@ -502,7 +559,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
 #pragma unroll
                 for ( int t = 0; t < NT; ++t )
 #pragma unroll
-                    for ( int r = 0; r < 4; ++r )
+                    for ( int r = 0; r < NR; ++r )
                         acc[t][r] = 0.0;
             }
         };
@@ -585,21 +642,38 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
 #pragma unroll
                     for ( int n = 0; n < 4; ++n )
                     {
-                        RC::put_pair( rp + 4 * n, wt[MF::QUAD][n], gt[MF::QUAD][n] );
-                        RC::put_pair( rp + 4 * ( SLIDE ? ( key + n ) & 3 : n ) + 2, wt[2][n],
-                                      gt[2][n] );
+                        if constexpr ( ORDER == 1 )
+                            RC::put_pair( rp + 2 * n, wt[2][n], gt[2][n] );
+                        else
+                        {
+                            RC::put_pair( rp + 4 * n, wt[MF::QUAD][n], gt[MF::QUAD][n] );
+                            RC::put_pair( rp + 4 * ( ( key + n ) & 3 ) + 2, wt[2][n], gt[2][n] );
+                        }
                     }
                     static_for<4>( [&]( auto S ) {
                         constexpr int sl = S;
                         Real v[ROW];
-                        v[0] = wt[MF::SLOT][sl];
-                        v[1] = gt[MF::SLOT][sl];
 #pragma unroll
-                        for ( int c = 2; c < ROW; ++c )
+                        for ( int c = 0; c < ROW; ++c )
                             v[c] = Real( 0 );
+                        if constexpr ( ORDER == 1 )
+                        {
+                            constexpr int i = sl >> 1, j = sl & 1;
+                            v[0] = wt[0][i] * wt[1][j];
+                            if constexpr ( TL::any_g() )
+                            {
+                                v[1] = gt[0][i] * wt[1][j];
+                                v[2] = wt[0][i] * gt[1][j];
+                            }
+                        }
+                        else
+                        {
+                            v[0] = wt[MF::SLOT][sl];
+                            v[1] = gt[MF::SLOT][sl];
+                        }
                         if constexpr ( TL::PAIR )
                         {
-                            v[2] = P[sl];
+                            v[TL::val( 0 )] = P[sl];
                             if constexpr ( NT == 2 && sl < 3 )
                                 slot_values<FL::v[FL::N - 1]>( P + 4, sl, v + TL::val( 1 ) );
                         }
@@ -609,7 +683,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                 constexpr int F = FL::v[t];
                                 if constexpr ( sl < ng_of( F ) )
                                     slot_values<F>( P + attr_of<FORMS...>( t ), sl,
-                                                    v + 2 + ( SHARED && t == 1 ? 1 : 0 ) );
+                                                    v + TL::val( 0 ) + ( SHARED && t == 1 ? 1 : 0 ) );
                             } );
                         RC::put_row( rp, sl, v );
                     } );
@@ -661,62 +735,86 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                             Step<Real, ROW> st[NS];
                             static_for<NS>( [&]( auto C ) {
                                 constexpr int c = C;
-                                st[c].xz = rp[4 * c * RS + l16];
-                                RC::get_row( rp + 4 * c * RS, slot, st[c].y );
+                                const Real* r = rp + 4 * c * RS;
+                                if constexpr ( ORDER == 1 )
+                                    RC::get_pair( r + 2 * kcol, st[c].xz, st[c].gz );
+                                else
+                                    st[c].xz = r[l16];
+                                RC::get_row( r, slot, st[c].y );
                             } );
                             __builtin_amdgcn_sched_barrier( 0 );
                             static_for<NS>( [&]( auto C ) {
                                 constexpr int c = C;
+                                Real wz, gz, A1, AQ, AS;
                                 // Particles past the group count zero.
-                                Real xz = st[c].xz;
-                                if ( c == NS - 1 )
-                                    xz = pslot < n - 4 * c ? xz : Real( 0 );
-                                const Real wq = quad_lane<0>( xz ), gq = quad_lane<1>( xz );
-                                const Real wz = quad_lane<2>( xz ), gz = quad_lane<3>( xz );
-                                const Real A1 = wq * st[c].y[0], AQ = gq * st[c].y[0],
-                                           AS = wq * st[c].y[1];
-                                Real B[NT][3];
-                                static_for<NT>( [&]( auto T ) {
-                                    constexpr int t = T;
-                                    const Real* v = st[c].y + TL::val( t );
-                                    if constexpr ( !TL::has_g( t ) )
-                                        B[t][0] = wz * v[0];
-                                    else
+                                const bool in = c < NS - 1 || pslot < n - 4 * c;
+                                const Real xz = in ? st[c].xz : Real( 0 );
+                                if constexpr ( ORDER == 1 )
+                                {
+                                    wz = xz;
+                                    gz = in ? st[c].gz : Real( 0 );
+                                    A1 = st[c].y[0];
+                                    if constexpr ( TL::any_g() )
                                     {
-                                        const Real* h = v + ( TL::has_v( t ) ? 1 : 0 );
-                                        B[t][0] = gz * h[2];
-                                        if constexpr ( TL::has_v( t ) )
-                                            B[t][0] += wz * v[0];
-                                        B[t][1] = wz * h[MF::QUAD];
-                                        B[t][2] = wz * h[MF::SLOT];
+                                        AQ = st[c].y[1];
+                                        AS = st[c].y[2];
                                     }
-                                } );
+                                }
+                                else
+                                {
+                                    const Real wq = quad_lane<0>( xz ), gq = quad_lane<1>( xz );
+                                    wz = quad_lane<2>( xz );
+                                    gz = quad_lane<3>( xz );
+                                    A1 = wq * st[c].y[0];
+                                    AQ = gq * st[c].y[0];
+                                    AS = wq * st[c].y[1];
+                                }
                                 static_for<NT>( [&]( auto T ) {
                                     constexpr int t = T;
-                                    constexpr int m1 = 1, m2 = F32 ? 2 : 1;
+                                    constexpr int m1 = ORDER > 1 ? 1 : 0;
+                                    constexpr int m2 = ORDER > 1 ? ( F32 ? 2 : 1 ) : 0;
+                                    constexpr int dq = ORDER > 1 ? MF::QUAD : 0;
+                                    constexpr int ds = ORDER > 1 ? MF::SLOT : 1;
+                                    const Real* v = st[c].y + TL::val( t );
+                                    const Real* h = v + ( TL::has_v( t ) ? 1 : 0 );
                                     if constexpr ( c == 0 )
                                     {
                                         D[t][0] = D[t][1] = D[t][2] = V4{ 0, 0, 0, 0 };
                                         if constexpr ( !F32 )
-                                            D[t][0] =
-                                                V4{ acc[t][0], acc[t][1], acc[t][2], acc[t][3] };
+                                        {
+#pragma unroll
+                                            for ( int r = 0; r < NR; ++r )
+                                                D[t][0][r] = acc[t][r];
+                                        }
                                     }
-                                    D[t][0] = MF::mac( A1, B[t][0], D[t][0] );
-                                    if constexpr ( TL::has_g( t ) )
+                                    auto mac = [&]( Real A, Real B, V4& d ) {
+                                        if constexpr ( ORDER == 1 )
+                                            d = mac4( A, B, d );
+                                        else
+                                            d = MF::mac( A, B, d );
+                                    };
+                                    if constexpr ( !TL::has_g( t ) )
+                                        mac( A1, wz * v[0], D[t][0] );
+                                    else
                                     {
-                                        D[t][m1] = MF::mac( AQ, B[t][1], D[t][m1] );
-                                        D[t][m2] = MF::mac( AS, B[t][2], D[t][m2] );
+                                        Real b1 = gz * h[2];
+                                        if constexpr ( TL::has_v( t ) )
+                                            b1 += wz * v[0];
+                                        mac( A1, b1, D[t][0] );
+                                        mac( AQ, wz * h[dq], D[t][m1] );
+                                        mac( AS, wz * h[ds], D[t][m2] );
                                     }
                                 } );
                             } );
                             static_for<NT>( [&]( auto T ) {
                                 constexpr int t = T;
+                                constexpr bool split = ORDER > 1 && TL::has_g( t );
 #pragma unroll
-                                for ( int r = 0; r < 4; ++r )
+                                for ( int r = 0; r < NR; ++r )
                                     if constexpr ( !F32 )
-                                        acc[t][r] = TL::has_g( t ) ? D[t][0][r] + D[t][1][r]
-                                                                   : D[t][0][r];
-                                    else if constexpr ( TL::has_g( t ) )
+                                        acc[t][r] =
+                                            split ? D[t][0][r] + D[t][1][r] : D[t][0][r];
+                                    else if constexpr ( split )
                                         acc[t][r] +=
                                             (double)( ( D[t][0][r] + D[t][1][r] ) + D[t][2][r] );
                                     else
