@@ -726,6 +726,7 @@ struct TileShape
 {
     int T[3];
     int cap;
+    int sub; // scatters: particles whose records are in LDS
 };
 
 // LDS bytes of the tiled kernels; mirrors their in-kernel layout.  vals: the
@@ -750,7 +751,7 @@ size_t tile_lds_bytes( TileKind kind, bool fp64, const int* slot_ng, int nslot, 
     for ( int i = 0; i < nslot; ++i )
         dt += slot_ng[i];
     b = a16( 8 * (size_t)dt * wn );
-    b = a16( b + real * ( SCATTER_BLOCK / 64 ) * ( scatter_sub( scatter_grad( vals ) ) + 3 ) *
+    b = a16( b + real * ( SCATTER_BLOCK / 64 ) * ( sh.sub + 3 ) *
                      scatter_record( fp64, order, scatter_row( order, vals ) ) );
     b = a16( b + 8 * runs );
     b = a16( b + 4 * ( runs + 1 ) );
@@ -776,7 +777,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
         bool found = false;
         for ( int c = 8; c >= 2; --c )
         {
-            TileShape sh = { { c, c, c }, 0 };
+            TileShape sh = { { c, c, c }, 0, 0 };
             if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, vals, order, sh ) >
                  (size_t)( fp64 ? 78 : 52 ) * 1024 )
                 continue;
@@ -798,6 +799,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
     const int extra = ( order == 1 ) ? 1 : 3;
     const int c = scatter_cells_k( order );
     const int waves = scatter_waves( fp64, scatter_grad( vals ) );
+    const int sub = scatter_sub( order, scatter_grad( vals ), nslot, mean_ppc );
     bool found = false;
     double best_bricks = 0.0;
     for ( int w = waves; w >= 2 && ( !found || best_bricks > 1048576.0 ); w = w > 2 ? 2 : 1 )
@@ -806,7 +808,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
         for ( int a = 2; a <= 8; ++a )
             for ( int b = a; b <= a + 1 && b <= 8; ++b )
             {
-                TileShape sh = { { a, b, c }, 0 };
+                TileShape sh = { { a, b, c }, 0, sub };
                 if ( tile_lds_bytes( kind, fp64, slot_ng, nslot, vals, order, sh ) >
                      (size_t)scatter_lds( w ) )
                     continue;
@@ -860,6 +862,7 @@ bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
     t.max_runs = sh.T[0] * sh.T[1];
     t.max_win_nodes = t.win[0] * t.win[1] * t.win[2];
     t.cap = sh.cap;
+    t.sub = sh.sub;
     t.bin_begin = bins->begin;
     // Window walk order: largest grid stride first.
     int perm[3] = { 0, 1, 2 };

@@ -352,6 +352,7 @@ struct TileArgs
     int32_t max_runs;            // tile[0] * tile[1]
     int32_t max_win_nodes;       // win[0] * win[1] * win[2]
     int32_t cap;                 // particles per part
+    int32_t sub;                 // particles of a scatter's records in LDS
     int32_t grid;                // workgroups launched (a multiple of 8)
     int64_t bin_begin;           // particle index of cell offset 0
     // Particle at each binned position q (perm[q - bin_begin]) when the
@@ -383,12 +384,21 @@ constexpr int scatter_waves( bool fp64, bool grad )
     return fp64 ? ( grad ? 2 : 3 ) : ( grad ? 3 : 4 );
 }
 constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
-// Particles of a wave's batch of 64 whose records are in LDS at a time.
-// Larger records leave the window too little room with 64 (and cost a wave per
-// SIMD); 16 break more groups apart: at 128^3 x 16 FP32 the MPM P2G takes
-// 1.51 ms with 32 and 1.67 ms with 16, and mass and momentum of 8.4 M clustered
-// particles, whose windows are larger, 0.50 ms with 32 and 0.46 ms with 16.
-constexpr int scatter_sub( bool grad ) { return grad ? 32 : 16; }
+// Particles of a wave's batch of 64 whose records are in LDS at a time.  16
+// leave the window more room (and cost a wave per SIMD with value terms if
+// they were 64), 32 break fewer runs of one cell apart.  Value terms take 16:
+// mass and momentum of 8.4 M clustered particles 0.46 ms against 0.50 ms.
+// Gradient terms take 32, the fused MPM P2G below SCATTER_SPARSE particles a
+// cell 16, in ms with 32 and with 16 (quadratic unless said):
+//   FP32, particles a cell:  2: 0.91 0.85   6: 0.48 0.44   16: 1.52 1.67
+//   FP64:  2: 1.28 1.16   3 (cubic): 0.72 0.61   4: 0.94 0.88   16: 1.24 1.38
+//   8 (cubic): 0.26 0.29
+// (linear splines, 2, FP64: 0.51 0.54; the G2P adjoint at 3: 0.40 0.42).
+constexpr double SCATTER_SPARSE = 6.0;
+constexpr int scatter_sub( int order, bool grad, int nslot, double mean_ppc )
+{
+    return !grad || ( order > 1 && nslot > 1 && mean_ppc < SCATTER_SPARSE ) ? 16 : 32;
+}
 // Cells of a scatter brick along k, a compile-time stride of the LDS window
 // (linear splines: groups of three cells).
 constexpr int scatter_cells_k( int order ) { return order == 1 ? 9 : 8; }

@@ -6,7 +6,8 @@
 //                        K^3 stencil loads, register accumulation.
 //   scatter_atomic_kernel P2G forward and G2P adjoint for particles in any
 //                        order: one thread per particle, global atomics.
-// The cell-sorted (tiled) variants live in ca_tiled.hip.
+// The cell-sorted (tiled) variants live in ca_tiled.hip (gathers)
+// and ca_scatter.hip.
 #include "ca_device.hpp"
 
 #include <utility>

@@ -438,7 +438,7 @@ struct Step
     Real y[ROW];
 };
 
-template <class Real, bool CONTIG, bool SHARED, int... FORMS>
+template <class Real, bool CONTIG, bool SHARED, int SUB, int... FORMS>
 __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 8, Tiles<SHARED, FORMS...>::any_g() ) ) ) void scatter_cells_kernel(
     ScatterArgs a, TileArgs ta )
 {
@@ -452,7 +452,6 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     constexpr int RS = RC::STRIDE;
     constexpr int NP = attr_len<FORMS...>();
     constexpr int NWAVE = SCATTER_BLOCK / 64;
-    constexpr int SUB = scatter_sub( TL::any_g() );
     constexpr int NR = acc_regs<Real>();
     constexpr bool F32 = sizeof( Real ) == 4;
     // Window nodes along k sit in column (node index mod 4), so that the
@@ -886,6 +885,12 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     }
 }
 
+template <int F>
+constexpr int single_sub()
+{
+    return scatter_sub( ORDER, Tiles<false, F>::any_g(), 1, 0.0 );
+}
+
 template <class Real, bool CONTIG>
 hipError_t scatter_cells_launch( int plan, const ScatterArgs& a, const TileArgs& t, size_t lds,
                                  hipStream_t s )
@@ -896,7 +901,7 @@ hipError_t scatter_cells_launch( int plan, const ScatterArgs& a, const TileArgs&
         {
 #define CA_CASE( F )                                                           \
     case F:                                                                    \
-        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, F>, a, t, lds, s, SCATTER_BLOCK );
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, single_sub<F>(), F>, a, t, lds, s, SCATTER_BLOCK );
             CA_CASE( FORM_SV )
             CA_CASE( FORM_VV )
             CA_CASE( FORM_SG )
@@ -909,14 +914,21 @@ hipError_t scatter_cells_launch( int plan, const ScatterArgs& a, const TileArgs&
         }
     }
     if ( plan == PLAN_MPM_P2G )
+    {
+        if constexpr ( ORDER > 1 )
+            if ( t.sub == 16 )
+                return launch_tile_kernel(
+                    scatter_cells_kernel<Real, CONTIG, false, 16, FORM_SV, FORM_VV, FORM_TD>, a, t,
+                    lds, s, SCATTER_BLOCK );
         return launch_tile_kernel(
-            scatter_cells_kernel<Real, CONTIG, false, FORM_SV, FORM_VV, FORM_TD>, a, t, lds, s,
+            scatter_cells_kernel<Real, CONTIG, false, 32, FORM_SV, FORM_VV, FORM_TD>, a, t, lds, s,
             SCATTER_BLOCK );
+    }
     if ( plan == PLAN_MASS_MOMENTUM )
-        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, FORM_SV, FORM_VV>,
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, false, 16, FORM_SV, FORM_VV>,
                                    a, t, lds, s, SCATTER_BLOCK );
     if ( plan == PLAN_MPM_G2P )
-        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, true, FORM_VV, FORM_TDT>,
+        return launch_tile_kernel( scatter_cells_kernel<Real, CONTIG, true, 32, FORM_VV, FORM_TDT>,
                                    a, t, lds, s, SCATTER_BLOCK );
     return hipErrorInvalidValue;
 }

@@ -16,6 +16,8 @@ pytestmark = pytest.mark.gpu
 
 POPULATION = [0, 1, 2, 3, 4, 5, 7, 8, 9, 0, 12, 13, 15, 16, 17, 20, 31, 32, 33, 48, 63, 64, 65,
               0, 0, 130]
+# Below 6 a cell, where the fused MPM P2G keeps the records of 16 particles.
+SPARSE = [0, 1, 2, 3, 4, 0, 0, 16, 17, 0, 0, 1, 33, 0, 0, 5]
 CELLS = (5, 7, 19)
 CELL = 0.5
 LOW = np.array([0.25, -1.0, 2.0])
@@ -23,11 +25,11 @@ SETS = [(0, 1, 4), (0, 1), (0,), (1,), (2,), (3,), (4,)]
 
 
 class Cloud:
-    def __init__(self, ca, oracle, seed, moved=0.0):
+    def __init__(self, ca, oracle, seed, moved=0.0, population=POPULATION):
         rng = np.random.default_rng(seed)
         cells = np.stack(np.meshgrid(*[np.arange(c) for c in CELLS], indexing="ij"), -1)
         cells = cells.reshape(-1, 3)
-        pop = np.resize(POPULATION, len(cells))
+        pop = np.resize(population, len(cells))
         cell_of = np.repeat(cells, pop, axis=0)
         self.n = len(cell_of)
         high = LOW + CELL * np.array(CELLS)
@@ -69,8 +71,9 @@ class Cloud:
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("order", [1, 2, 3])
 @pytest.mark.parametrize("moved", [0.0, 0.4])
-def test_group_sizes(ca, oracle, order, dtype, moved):
-    c = Cloud(ca, oracle, 31 + order, moved)
+@pytest.mark.parametrize("population", [POPULATION, SPARSE], ids=["dense", "sparse"])
+def test_group_sizes(ca, oracle, order, dtype, moved, population):
+    c = Cloud(ca, oracle, 31 + order, moved, population)
     own = c.mesh.owned_slices()
     ref = {op: c.reference(oracle, op, order, dtype) for op in range(5)}
     for ops in SETS:
