@@ -1164,8 +1164,8 @@ cabana_amd_status validate_bins( cabana_amd_context* ctx,
 
 // The drop-in call shape passes no binning.  Then, for the orders with
 // cell-tiled kernels, the library bins the particles itself: owned-cell
-// keys, the stable radix sort of cabana_amd_linked_cell_build, counts and
-// offsets, kept in SLOT_BINS with the sorted order as a permutation that
+// keys, the stable radix sort of cabana_amd_linked_cell_build (or a count by
+// cell where that is faster), counts and offsets, kept in SLOT_BINS with the sorted order as a permutation that
 // the tiled kernels read particles through (the particles stay where they
 // are).  `bins` is left as it is when the call passed one, when the
 // context has the feature off, or when it cannot apply.
@@ -1201,12 +1201,12 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     int digit_bits;
     lcl_sort_passes( key_bits, &digit_bits );
     const int64_t nhist = ( (int64_t)1 << digit_bits ) * lcl_sort_tiles( n );
-    const int64_t nscan = nhist > ncell ? nhist : ncell;
-    const int64_t nblock = ( nscan + 1023 ) / 1024 + 1;
+    const int64_t nblock = ( ncell + 1023 ) / 1024 + 1;
     const int64_t nkey = n + 64;
     CA_HIP( ctx, ctx->ensure( SLOT_CELL_OF, sizeof( int32_t ) * 4 * nkey ), "scratch" );
     CA_HIP( ctx,
-            ctx->ensure( SLOT_CURSOR, ( sizeof( int64_t ) + sizeof( int32_t ) ) * ( nhist + 64 ) ),
+            ctx->ensure( SLOT_CURSOR,
+                         sizeof( int64_t ) * SORT_MAX_DIGITS + sizeof( int32_t ) * nhist ),
             "scratch" );
     CA_HIP( ctx, ctx->ensure( SLOT_SCAN, sizeof( int64_t ) * nblock ), "scratch" );
     const size_t o_off = a16( sizeof( int32_t ) * (size_t)ncell );
@@ -1217,8 +1217,8 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     int64_t* offsets = reinterpret_cast<int64_t*>( base + o_off );
     int64_t* perm = reinterpret_cast<int64_t*>( base + o_perm );
     int32_t* keys = static_cast<int32_t*>( ctx->scratch[SLOT_CELL_OF] );
-    int64_t* digit_base = static_cast<int64_t*>( ctx->scratch[SLOT_CURSOR] );
-    int32_t* hist = reinterpret_cast<int32_t*>( digit_base + nhist + 64 );
+    int64_t* totals = static_cast<int64_t*>( ctx->scratch[SLOT_CURSOR] );
+    int32_t* hist = reinterpret_cast<int32_t*>( totals + SORT_MAX_DIGITS );
     int64_t* sums = static_cast<int64_t*>( ctx->scratch[SLOT_SCAN] );
     if ( !ctx->deterministic && auto_bin_counts( n, ncell ) )
     {
@@ -1230,7 +1230,7 @@ cabana_amd_status build_library_bins( cabana_amd_context* ctx, const MeshDev& m,
     else
     {
         const SortScratch w = { keys, keys + nkey, keys + 2 * nkey, keys + 3 * nkey,
-                                hist, digit_base, sums, nblock };
+                                hist, totals };
         CA_HIP( ctx,
                 launch_auto_bin_sort( *ctx, pts, n, m, key_bits, w, perm, ncell, counts, offsets, s ),
                 "bin sort" );
@@ -2330,26 +2330,22 @@ extern "C" cabana_amd_status cabana_amd_linked_cell_build(
     int digit_bits;
     lcl_sort_passes( key_bits, &digit_bits );
     const int64_t nhist = ( (int64_t)1 << digit_bits ) * lcl_sort_tiles( np );
-    const int64_t nblock = ( nhist + 1023 ) / 1024 + 1;
     const int64_t nkey = np + 64;
     CA_HIP( ctx, ctx->ensure( SLOT_CELL_OF, sizeof( int32_t ) * 4 * nkey ),
             "scratch" );
     CA_HIP( ctx,
             ctx->ensure( SLOT_CURSOR,
-                         ( sizeof( int64_t ) + sizeof( int32_t ) ) * ( nhist + 64 ) ),
-            "scratch" );
-    CA_HIP( ctx, ctx->ensure( SLOT_SCAN, sizeof( int64_t ) * nblock ),
+                         sizeof( int64_t ) * SORT_MAX_DIGITS + sizeof( int32_t ) * nhist ),
             "scratch" );
     int32_t* keys = static_cast<int32_t*>( ctx->scratch[SLOT_CELL_OF] );
-    int64_t* digit_base = static_cast<int64_t*>( ctx->scratch[SLOT_CURSOR] );
-    int32_t* hist = reinterpret_cast<int32_t*>( digit_base + nhist + 64 );
-    int64_t* sums = static_cast<int64_t*>( ctx->scratch[SLOT_SCAN] );
+    int64_t* totals = static_cast<int64_t*>( ctx->scratch[SLOT_CURSOR] );
+    int32_t* hist = reinterpret_cast<int32_t*>( totals + SORT_MAX_DIGITS );
     CA_HIP( ctx,
             launch_fill_i32( *ctx, reinterpret_cast<int32_t*>( ctx->bad ), 2, 0,
                              s ),
             "fill" );
     const SortScratch w = { keys, keys + nkey, keys + 2 * nkey, keys + 3 * nkey,
-                            hist, digit_base, sums, nblock };
+                            hist, totals };
     CA_HIP( ctx,
             launch_lcl_build( *ctx, pos, begin, np, g, (int32_t)ncell, ctx->bad, key_bits, w,
                               permutes, ncell, counts, offsets, s ),

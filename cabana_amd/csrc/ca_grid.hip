@@ -274,16 +274,6 @@ struct OwnedKey
     __device__ int32_t operator()( int64_t p ) const { return owned_cell( pos, p, m ); }
 };
 
-// Keys of particles [begin, end).
-template <class Key>
-__global__ __launch_bounds__( BLOCK ) void bin_key_kernel( Key key, int64_t begin, int64_t end,
-                                                           int32_t* keys )
-{
-    const int64_t p = begin + (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-    if ( p < end )
-        keys[p - begin] = key( p );
-}
-
 constexpr int SCAN_BLOCK = 1024;
 
 __global__ __launch_bounds__( SCAN_BLOCK ) void scan_reduce_kernel(
@@ -460,8 +450,10 @@ __global__ __launch_bounds__( SCAN_BLOCK ) void scan_apply_kernel(
 // A tile of RS_TILE keys belongs to one workgroup; wave w owns the contiguous
 // run [w * 64 * RS_ITEMS, (w + 1) * 64 * RS_ITEMS) of its tile and walks it
 // 64 keys at a time, so (wave, step, lane) is index order.  Pass layout:
-//   hist:    per-tile digit counts, digit-major: hist[digit * ntiles + tile];
-//   scan:    exclusive scan of hist gives every (digit, tile) its output base;
+//   hist:    per-tile digit counts, digit-major: hist[digit * ntiles + tile]
+//            (the first pass counts the keys as they are formed);
+//   rows:    exclusive scan of every digit's row, one workgroup each; the
+//            digits' totals are scanned by every workgroup of the scatter;
 //   scatter: each key's rank among equal digits of its tile (ballot peers +
 //            per-wave running counts in LDS), a tile-local reorder in LDS,
 //            then writes in tile order, so equal digits leave contiguously.
@@ -473,10 +465,40 @@ constexpr int RS_WAVES = RS_BLOCK / 64;
 constexpr int RS_MAX_BITS = 8;
 constexpr int RS_MAX_BINS = 1 << RS_MAX_BITS;
 static_assert( RS_MAX_BINS == RS_BLOCK, "one digit per thread in the scans" );
+static_assert( RS_MAX_BINS == SORT_MAX_DIGITS, "the totals' scratch" );
 
 __global__ __launch_bounds__( RS_BLOCK ) void radix_hist_kernel(
     const int32_t* keys, int64_t n, int shift, int nbins, int64_t ntiles,
     int32_t* hist )
+{
+    __shared__ uint32_t h[RS_MAX_BINS];
+    h[threadIdx.x] = 0;
+    __syncthreads();
+    const int64_t t0 = (int64_t)blockIdx.x * RS_TILE;
+    const uint32_t mask = (uint32_t)nbins - 1u;
+    uint32_t key[RS_ITEMS];
+#pragma unroll
+    for ( int k = 0; k < RS_ITEMS; ++k )
+    {
+        const int64_t i = t0 + k * RS_BLOCK + threadIdx.x;
+        key[k] = i < n ? (uint32_t)keys[i] : 0u;
+    }
+#pragma unroll
+    for ( int k = 0; k < RS_ITEMS; ++k )
+        if ( t0 + k * RS_BLOCK + threadIdx.x < n )
+            atomicAdd( &h[( key[k] >> shift ) & mask], 1u );
+    __syncthreads();
+    if ( (int)threadIdx.x < nbins )
+        hist[threadIdx.x * ntiles + blockIdx.x] = (int32_t)h[threadIdx.x];
+}
+
+// Keys of particles [begin, begin + n) and their digit counts for the first
+// pass.
+template <class Key>
+__global__ __launch_bounds__( RS_BLOCK ) void bin_key_hist_kernel( Key key, int64_t begin,
+                                                                   int64_t n, int nbins,
+                                                                   int64_t ntiles, int32_t* keys,
+                                                                   int32_t* hist )
 {
     __shared__ uint32_t h[RS_MAX_BINS];
     h[threadIdx.x] = 0;
@@ -488,11 +510,27 @@ __global__ __launch_bounds__( RS_BLOCK ) void radix_hist_kernel(
     {
         const int64_t i = t0 + k * RS_BLOCK + threadIdx.x;
         if ( i < n )
-            atomicAdd( &h[( (uint32_t)keys[i] >> shift ) & mask], 1u );
+        {
+            const int32_t x = key( begin + i );
+            keys[i] = x;
+            atomicAdd( &h[(uint32_t)x & mask], 1u );
+        }
     }
     __syncthreads();
     if ( (int)threadIdx.x < nbins )
         hist[threadIdx.x * ntiles + blockIdx.x] = (int32_t)h[threadIdx.x];
+}
+
+// Exclusive scan of a digit's row in place (a round's reads precede its
+// writes, and the rounds are disjoint), and its total.
+__global__ __launch_bounds__( SCAN_BLOCK ) void radix_rows_kernel( int32_t* hist, int64_t ntiles,
+                                                                   int64_t* totals )
+{
+    int32_t* row = hist + blockIdx.x * ntiles;
+    const int64_t total =
+        scan_one( row, (int)ntiles, [&]( int i, int32_t, int64_t before ) { row[i] = (int32_t)before; } );
+    if ( threadIdx.x == 0 )
+        totals[blockIdx.x] = total;
 }
 
 // Exclusive scan of one value per thread over the workgroup; returns the
@@ -530,19 +568,27 @@ __device__ __forceinline__ uint32_t rs_block_scan( uint32_t v, uint32_t* wsum,
 template <bool FIRST, bool LAST>
 __global__ __launch_bounds__( RS_BLOCK ) void radix_scatter_kernel(
     const int32_t* keys_in, const int32_t* vals_in, int64_t n, int shift,
-    int nbins, int64_t ntiles, const int64_t* digit_base, int32_t* keys_out,
-    int32_t* vals_out, int64_t* perm_out, int64_t begin )
+    int nbins, int64_t ntiles, const int32_t* hist, const int64_t* totals,
+    int32_t* keys_out, int32_t* vals_out, int64_t* perm_out, int64_t begin )
 {
     __shared__ uint32_t wcnt[RS_WAVES][RS_MAX_BINS];
     __shared__ uint32_t tstart[RS_MAX_BINS];
     __shared__ int64_t gadj[RS_MAX_BINS];
-    __shared__ uint32_t wsum[RS_WAVES];
+    __shared__ uint32_t wsum[2][RS_WAVES];
     __shared__ int32_t lkey[RS_TILE];
     __shared__ int32_t lval[RS_TILE];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for ( int q = 0; q < RS_WAVES; ++q )
         wcnt[q][threadIdx.x] = 0;
+    // First output position of the tile's keys of digit threadIdx.x.
+    int64_t obase = 0;
+    {
+        const int d = threadIdx.x;
+        uint32_t all;
+        const uint32_t before = d < nbins ? (uint32_t)hist[(int64_t)d * ntiles + blockIdx.x] : 0u;
+        obase = (int64_t)rs_block_scan( d < nbins ? (uint32_t)totals[d] : 0u, wsum[0], &all ) + before;
+    }
     __syncthreads();
     const int64_t t0 = (int64_t)blockIdx.x * RS_TILE;
     const int64_t wbase = t0 + (int64_t)w * 64 * RS_ITEMS;
@@ -599,10 +645,9 @@ __global__ __launch_bounds__( RS_BLOCK ) void radix_scatter_kernel(
             run += c;
         }
         uint32_t total;
-        const uint32_t st = rs_block_scan( d < nbins ? run : 0u, wsum, &total );
+        const uint32_t st = rs_block_scan( d < nbins ? run : 0u, wsum[1], &total );
         tstart[d] = st;
-        gadj[d] = d < nbins ? digit_base[(int64_t)d * ntiles + blockIdx.x] - st
-                            : 0;
+        gadj[d] = obase - st;
     }
     __syncthreads();
 #pragma unroll
@@ -1399,13 +1444,13 @@ hipError_t bin_sort( Launcher& L, const char* name, const Key& key, int64_t begi
         return launch_lcl_bounds( L, w.keys_b, n, ncell, counts, offsets, s );
     }
     L.before( name, s );
-    hipLaunchKernelGGL( bin_key_kernel<Key>, blocks_for( n ), dim3( BLOCK ), 0, s, key, begin,
-                        begin + n, w.keys_a );
-    L.after( name, s );
     int32_t* hist = w.hist;
-    int64_t* digit_base = w.digit_base;
+    int64_t* totals = w.totals;
     const int nbins = 1 << dbits;
     const int64_t ntiles = lcl_sort_tiles( n );
+    hipLaunchKernelGGL( bin_key_hist_kernel<Key>, dim3( (unsigned)ntiles ), dim3( RS_BLOCK ), 0, s, key,
+                        begin, n, nbins, ntiles, w.keys_a, hist );
+    L.after( name, s );
     int32_t* kin = w.keys_a;
     int32_t* kout = w.keys_b;
     int32_t* vin = w.vals_a;
@@ -1413,40 +1458,42 @@ hipError_t bin_sort( Launcher& L, const char* name, const Key& key, int64_t begi
     for ( int p = 0; p < passes; ++p )
     {
         const int shift = p * dbits;
-        L.before( "lcl_sort_hist", s );
-        hipLaunchKernelGGL( radix_hist_kernel, dim3( (unsigned)ntiles ),
-                            dim3( RS_BLOCK ), 0, s, kin, n, shift, nbins,
-                            ntiles, hist );
-        L.after( "lcl_sort_hist", s );
-        hipError_t e = launch_exclusive_scan( L, hist, digit_base,
-                                              (int64_t)nbins * ntiles,
-                                              w.block_sums, w.nblock_cap, s );
-        if ( e != hipSuccess )
-            return e;
+        if ( p > 0 )
+        {
+            L.before( "lcl_sort_hist", s );
+            hipLaunchKernelGGL( radix_hist_kernel, dim3( (unsigned)ntiles ),
+                                dim3( RS_BLOCK ), 0, s, kin, n, shift, nbins,
+                                ntiles, hist );
+            L.after( "lcl_sort_hist", s );
+        }
+        L.before( "lcl_sort_rows", s );
+        hipLaunchKernelGGL( radix_rows_kernel, dim3( (unsigned)nbins ), dim3( SCAN_BLOCK ), 0, s,
+                            hist, ntiles, totals );
+        L.after( "lcl_sort_rows", s );
         const bool first = p == 0, last = p == passes - 1;
         L.before( "lcl_sort_scatter", s );
         if ( first && last )
             hipLaunchKernelGGL( ( radix_scatter_kernel<true, true> ),
                                 dim3( (unsigned)ntiles ), dim3( RS_BLOCK ), 0,
                                 s, kin, vin, n, shift, nbins, ntiles,
-                                digit_base, kout, vout, permutes, begin );
+                                hist, totals, kout, vout, permutes, begin );
         else if ( first )
             hipLaunchKernelGGL( ( radix_scatter_kernel<true, false> ),
                                 dim3( (unsigned)ntiles ), dim3( RS_BLOCK ), 0,
                                 s, kin, vin, n, shift, nbins, ntiles,
-                                digit_base, kout, vout, permutes, begin );
+                                hist, totals, kout, vout, permutes, begin );
         else if ( last )
             hipLaunchKernelGGL( ( radix_scatter_kernel<false, true> ),
                                 dim3( (unsigned)ntiles ), dim3( RS_BLOCK ), 0,
                                 s, kin, vin, n, shift, nbins, ntiles,
-                                digit_base, kout, vout, permutes, begin );
+                                hist, totals, kout, vout, permutes, begin );
         else
             hipLaunchKernelGGL( ( radix_scatter_kernel<false, false> ),
                                 dim3( (unsigned)ntiles ), dim3( RS_BLOCK ), 0,
                                 s, kin, vin, n, shift, nbins, ntiles,
-                                digit_base, kout, vout, permutes, begin );
+                                hist, totals, kout, vout, permutes, begin );
         L.after( "lcl_sort_scatter", s );
-        e = hipGetLastError();
+        const hipError_t e = hipGetLastError();
         if ( e != hipSuccess )
             return e;
         int32_t* t = kin;

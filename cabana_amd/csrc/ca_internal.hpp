@@ -496,8 +496,9 @@ hipError_t launch_exclusive_scan( Launcher& L, const int32_t* in, int64_t* out,
                                   int64_t n, int64_t* block_sums,
                                   int64_t nblock_cap, hipStream_t s );
 // Scratch of a sorting build of n particles: keys and values of two buffers
-// (n + 64 int32 each), hist (int32) and digit_base (int64) of 2^digit_bits *
-// lcl_sort_tiles( n ) + 64 entries, block sums of the scans.
+// (n + 64 int32 each), hist of 2^digit_bits * lcl_sort_tiles( n ) int32 and
+// the totals of SORT_MAX_DIGITS digits.
+constexpr int SORT_MAX_DIGITS = 256;
 struct SortScratch
 {
     int32_t* keys_a;
@@ -505,9 +506,7 @@ struct SortScratch
     int32_t* vals_a;
     int32_t* vals_b;
     int32_t* hist;
-    int64_t* digit_base;
-    int64_t* block_sums;
-    int64_t nblock_cap;
+    int64_t* totals;
 };
 int64_t lcl_sort_tiles( int64_t n );
 int lcl_sort_passes( int key_bits, int* digit_bits );
