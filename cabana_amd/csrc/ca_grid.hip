@@ -1867,12 +1867,14 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
 }
 
 // Counting needs four launches against the sort's three a pass, but its
-// atomics reach about 24 G/s on random particles: 262144 particles on 32^3
-// cells take 41 us against 95 us, 2.1 M on 64^3 cells 137 against 150, and the
-// sort is ahead beyond.  Few cells would contend for their counters.
+// atomics reach about 24 G/s on random particles.  P2G and G2P of mass and
+// momentum, unbinned, counting and sorting: 262144 particles on 32^3 cells 134
+// and 177 us, 1.06 M on 51^3 cells 336 and 350, 1.56 M on 58^3 cells 471 and
+// 446, 2.1 M on 64^3 cells 577 and 497.  Few cells would contend for their
+// counters.
 bool auto_bin_counts( int64_t n, int64_t ncell )
 {
-    return n > RS_SMALL_MAX && n <= ( 1 << 21 ) + ( 1 << 16 ) && n / ncell <= 64;
+    return n > RS_SMALL_MAX && n <= ( 1 << 20 ) + ( 1 << 17 ) && n / ncell <= 64;
 }
 
 } // namespace cabana_amd

@@ -493,7 +493,7 @@ cabana_amd_status cabana_amd_particle_migrate(
 /* Calls that pass no binning (bins NULL, the drop-in shape of Cabana's p2g
  * and g2p) with spline orders 1 to 3 bin the particles by owned cell
  * themselves on the call's stream (cell keys, a stable radix sort or, up to
- * about 2^21 particles, a count by cell; in context scratch) and run the
+ * about 2^20 particles, a count by cell; in context scratch) and run the
  * cell-tiled kernels, reading
  * the particles in cell order through the sorted permutation; the
  * particles are not moved.  Results are those of the per-particle path up

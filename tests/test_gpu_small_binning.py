@@ -33,6 +33,22 @@ def test_build_matches_a_stable_sort(ca, n, dims, crowded):
     assert np.array_equal(lcl.offsets.cpu().numpy(), np.cumsum(counts) - counts)
 
 
+# Tiles of 4096 keys: a ragged last one, and one past the 8192 tiles that a
+# round of the digit rows' scan takes.
+@pytest.mark.parametrize("n", [40961, 8192 * 4096 + 4097])
+def test_tiled_sort(ca, n):
+    dims = (16, 11, 9)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x = torch.rand(n, 3, dtype=torch.float64, device="cuda", generator=g)
+    x *= torch.tensor(dims, dtype=torch.float64, device="cuda")
+    lcl = ca.createLinkedCellList(x, [1.0] * 3, [0.0] * 3, [float(d) for d in dims])
+    c = x.floor().long()
+    key = (c[:, 0] * dims[1] + c[:, 1]) * dims[2] + c[:, 2]
+    assert torch.equal(lcl.permutes, torch.sort(key, stable=True).indices)
+    counts = torch.bincount(key, minlength=dims[0] * dims[1] * dims[2])
+    assert torch.equal(lcl.counts.long().reshape(-1), counts)
+
+
 @pytest.mark.parametrize("n,cells", [(16384, 8), (16385, 8), (40000, 8), (40000, 24), (33000, 8)])
 @pytest.mark.parametrize("order", [1, 2])
 @pytest.mark.parametrize("cell_order", [False, True])
