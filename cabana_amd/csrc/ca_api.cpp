@@ -794,8 +794,11 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
     }
     // Scatters: the brick with the most cells per window node (fewest grid
     // atomics per cell) whose LDS lets a full set of workgroups run on a CU,
-    // among those that give every CU several bricks.  Above 2^20 bricks, where
-    // the part table itself is large, two workgroups per CU.
+    // among those that give every CU two bricks: MPM P2G of 32^3 cells x 8,
+    // FP32, takes 53 us with at least 1024 bricks (whose windows add more nodes
+    // to the grid, each rounded to FP32), 43 us with 512 and 48 us with 256.
+    // Above 2^20 bricks, where the part table itself is large, two workgroups
+    // per CU.
     const int extra = ( order == 1 ) ? 1 : 3;
     const int c = scatter_cells_k( order );
     const int waves = scatter_waves( fp64, scatter_grad( vals ) );
@@ -814,7 +817,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
                     continue;
                 const double bricks = bricks_of( sh );
                 const double share = (double)( a * b ) / ( ( a + extra ) * ( b + extra ) );
-                const double score = share * ( bricks < 1024.0 ? bricks / 1024.0 : 1.0 );
+                const double score = share * ( bricks < 512.0 ? bricks / 512.0 : 1.0 );
                 if ( score <= best )
                     continue;
                 best = score;
