@@ -770,8 +770,8 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                 }
                                 static_for<NT>( [&]( auto T ) {
                                     constexpr int t = T;
-                                    constexpr int m1 = ORDER > 1 ? 1 : 0;
-                                    constexpr int m2 = ORDER > 1 ? ( F32 ? 2 : 1 ) : 0;
+                                    constexpr int m1 = ORDER > 1 || !F32 ? 1 : 0;
+                                    constexpr int m2 = ORDER > 1 ? ( F32 ? 2 : 1 ) : ( F32 ? 0 : 2 );
                                     constexpr int dq = ORDER > 1 ? MF::QUAD : 0;
                                     constexpr int ds = ORDER > 1 ? MF::SLOT : 1;
                                     const Real* v = st[c].y + TL::val( t );
@@ -779,7 +779,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                     if constexpr ( c == 0 )
                                     {
                                         D[t][0] = D[t][1] = D[t][2] = V4{ 0, 0, 0, 0 };
-                                        if constexpr ( !F32 )
+                                        if constexpr ( !F32 && ORDER > 1 )
                                         {
 #pragma unroll
                                             for ( int r = 0; r < NR; ++r )
@@ -807,10 +807,17 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                             } );
                             static_for<NT>( [&]( auto T ) {
                                 constexpr int t = T;
-                                constexpr bool split = ORDER > 1 && TL::has_g( t );
+                                constexpr bool split = ( ORDER > 1 || !F32 ) && TL::has_g( t );
 #pragma unroll
                                 for ( int r = 0; r < NR; ++r )
-                                    if constexpr ( !F32 )
+                                    if constexpr ( !F32 && ORDER == 1 )
+                                        // (Chunks summed apart: one chain over
+                                        // the groups of three cells measured
+                                        // 1.1 to 1.2 times the error.)
+                                        acc[t][r] +=
+                                            split ? ( D[t][0][r] + D[t][1][r] ) + D[t][2][r]
+                                                  : D[t][0][r];
+                                    else if constexpr ( !F32 )
                                         acc[t][r] =
                                             split ? D[t][0][r] + D[t][1][r] : D[t][0][r];
                                     else if constexpr ( split )
