@@ -458,6 +458,10 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     // window slides to the next cell without moving the accumulators.  (The
     // windows of the linear spline are three cells apart and do not slide.)
     constexpr bool SLIDE = ORDER != 1;
+    // Steps of a chunk at most: the fused passes of sparse particles (records of
+    // 16) seldom have more than eight in a group, and chunks of four cost them
+    // 32 spilled registers.
+    constexpr int MAX_STEPS = SUB == 16 && TL::any_g() ? 2 : 4;
     extern __shared__ __align__( 16 ) unsigned char smem[];
 
     // LDS: the FP64 node window (one block per tile, [node][dof]), the waves'
@@ -484,7 +488,9 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     for ( int e = lane; e < RS * ( SUB + 3 ); e += 64 )
         rec[e] = Real( 0 );
 
-    const Real vmax = Real( sizeof( Real ) == 8 ? 1e300 : 1e30 ) /
+    // A thirty-second of the largest value: no sum of 16 products overflows
+    // where the values do not.
+    const Real vmax = Real( sizeof( Real ) == 8 ? 5.6e306 : 1.06e37 ) /
                       ( Real( 1 ) + (Real)a.mesh.rdx[0] + (Real)a.mesh.rdx[1] + (Real)a.mesh.rdx[2] );
 
     const PartLoop pl( ta );
@@ -720,14 +726,19 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                     s = e;
                     while ( n > 0 )
                     {
-                        // FP32 products are summed over 16 particles at most,
-                        // a gradient-type tile's three kinds apart, and the
-                        // sums added in FP64 (one FP32 sum of all three was
-                        // less accurate than the kernel before this one; its
-                        // products also wait for each other).  Each count of
-                        // steps is code of its own, without branches, so that
-                        // its operand reads are issued together: 1.87 -> 1.62
-                        // ms against a loop that read a step ahead.
+                        // FP32 products are summed over 8 particles at most for
+                        // a value-type tile and over 16 for a gradient-type
+                        // one, its three kinds apart, and the sums added in
+                        // FP64.  (Linear splines sum the three kinds in one
+                        // chain, but a lane's chain is of one particle a step,
+                        // 12 products at most.)  Relative L2 error of
+                        // momentum, 64^3 cells, quadratic, at 2, 8 and 16
+                        // particles a cell, e-8: 8.8 9.6 9.7; with chains of 16:
+                        // 8.8 9.9 10.5; the kernel before this one: 8.9 9.7
+                        // 10.3.  Each count of steps is code of its own, without
+                        // branches, so that its operand reads are issued
+                        // together: 1.87 -> 1.62 ms against a loop that read a
+                        // step ahead.
                         auto chunk = [&]( auto STEPS ) {
                             constexpr int NS = STEPS;
                             V4 D[NT][3];
@@ -777,15 +788,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                     const Real* v = st[c].y + TL::val( t );
                                     const Real* h = v + ( TL::has_v( t ) ? 1 : 0 );
                                     if constexpr ( c == 0 )
-                                    {
                                         D[t][0] = D[t][1] = D[t][2] = V4{ 0, 0, 0, 0 };
-                                        if constexpr ( !F32 && ORDER > 1 )
-                                        {
-#pragma unroll
-                                            for ( int r = 0; r < NR; ++r )
-                                                D[t][0][r] = acc[t][r];
-                                        }
-                                    }
                                     auto mac = [&]( Real A, Real B, V4& d ) {
                                         if constexpr ( ORDER == 1 )
                                             d = mac4( A, B, d );
@@ -803,40 +806,53 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                         mac( AQ, wz * h[dq], D[t][m1] );
                                         mac( AS, wz * h[ds], D[t][m2] );
                                     }
+                                    constexpr bool split = ( ORDER > 1 || !F32 ) && TL::has_g( t );
+                                    constexpr int CHAIN = F32 && !TL::has_g( t ) ? 2 : 4;
+                                    if constexpr ( c % CHAIN == CHAIN - 1 || c == NS - 1 )
+                                    {
+#pragma unroll
+                                        for ( int r = 0; r < NR; ++r )
+                                            if constexpr ( !F32 )
+                                            {
+                                                // (Chunks summed apart: one chain
+                                                // over all groups of a window
+                                                // measured up to 1.2 times the
+                                                // error.)
+                                                if constexpr ( !split )
+                                                    acc[t][r] += D[t][0][r];
+                                                else if constexpr ( ORDER == 1 )
+                                                    acc[t][r] += ( D[t][0][r] + D[t][1][r] ) + D[t][2][r];
+                                                else
+                                                    acc[t][r] += D[t][0][r] + D[t][1][r];
+                                            }
+                                            else if constexpr ( split && NS == 1 )
+                                                // Few particles: the roundings of
+                                                // the sum of the three kinds
+                                                // would be most of the error.
+                                                acc[t][r] +=
+                                                    ( (double)D[t][0][r] + (double)D[t][1][r] ) +
+                                                    (double)D[t][2][r];
+                                            else if constexpr ( split )
+                                                acc[t][r] += (double)( ( D[t][0][r] + D[t][1][r] ) +
+                                                                       D[t][2][r] );
+                                            else
+                                                acc[t][r] += (double)D[t][0][r];
+                                        if constexpr ( c < NS - 1 )
+                                            D[t][0] = V4{ 0, 0, 0, 0 };
+                                    }
                                 } );
                             } );
-                            static_for<NT>( [&]( auto T ) {
-                                constexpr int t = T;
-                                constexpr bool split = ( ORDER > 1 || !F32 ) && TL::has_g( t );
-#pragma unroll
-                                for ( int r = 0; r < NR; ++r )
-                                    if constexpr ( !F32 && ORDER == 1 )
-                                        // (Chunks summed apart: one chain over
-                                        // the groups of three cells measured
-                                        // 1.1 to 1.2 times the error.)
-                                        acc[t][r] +=
-                                            split ? ( D[t][0][r] + D[t][1][r] ) + D[t][2][r]
-                                                  : D[t][0][r];
-                                    else if constexpr ( !F32 )
-                                        acc[t][r] =
-                                            split ? D[t][0][r] + D[t][1][r] : D[t][0][r];
-                                    else if constexpr ( split )
-                                        acc[t][r] +=
-                                            (double)( ( D[t][0][r] + D[t][1][r] ) + D[t][2][r] );
-                                    else
-                                        acc[t][r] += (double)D[t][0][r];
-                            } );
                         };
-                        if ( n > 12 )
+                        if ( MAX_STEPS == 4 && n > 12 )
                             chunk( std::integral_constant<int, 4>{} );
-                        else if ( n > 8 )
+                        else if ( MAX_STEPS == 4 && n > 8 )
                             chunk( std::integral_constant<int, 3>{} );
                         else if ( n > 4 )
                             chunk( std::integral_constant<int, 2>{} );
                         else
                             chunk( std::integral_constant<int, 1>{} );
-                        n -= 16;
-                        rp += 16 * RS;
+                        n -= 4 * MAX_STEPS;
+                        rp += 4 * MAX_STEPS * RS;
                     }
                 }
                 // The records are rewritten by the next sub-batch.

@@ -97,3 +97,52 @@ def test_values_that_are_not_finite(ca, oracle, order, dtype):
             assert not fine.all() and fine.mean() > 0.3
             assert np.array_equal(fine, np.isfinite(got[own]))
             assert rel_l2(got[own][fine], ref[fine]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("terms", [(0,), (1,), (0, 1), (0, 1, 4)])
+@pytest.mark.parametrize("order", [1, 2])
+def test_fp32_value_sums_span_eight_particles(ca, order, terms):
+    """16 particles at one point whose weights are powers of two (times three):
+    the first of value 2^24, the last eight of value 1.  FP32 sums of eight
+    particles and FP64 sums of those are exact, and 2^24 + 8 is an FP32 number;
+    one FP32 chain of 16 would lose the eight ones."""
+    lg = ca.createLocalGrid(ca.createGlobalGrid(
+        ca.createUniformGlobalMesh([0.0] * 3, [8.0] * 3, 1.0), [True] * 3), 1)
+    at = 3.5 if order == 1 else 4.0
+    pts = torch.full((16, 3), at, dtype=torch.float64, device="cuda")
+    v = torch.zeros(16, 9, dtype=torch.float32, device="cuda")
+    v[0], v[8:] = 2.0 ** 24, 1.0
+    arrays, fs = [], []
+    for op in terms:
+        n, dofs = P2G_SHAPE[op]
+        arrays.append(ca.createArray("g", ca.createArrayLayout(lg, dofs, ca.Node()),
+                                     dtype=torch.float32))
+        value = torch.zeros_like(v) if op == 4 else v[:, :n].contiguous()
+        value = value.reshape((16,) if n == 1 else (16, 3) if n == 3 else (16, 3, 3))
+        fs.append(getattr(ca, P2G_FACTORY[op])(value, 1.0))
+    halo = ca.createHalo(ca.NodeHaloPattern(), 1, arrays[0])
+    bins = ca.createLinkedCellList(pts, [1.0] * 3, [0.0] * 3, [8.0] * 3)
+    ca.p2g(fs, pts, 16, ca.Spline(order), halo, arrays, bins=bins)
+    w = torch.tensor([0.5, 0.5] if order == 1 else [0.125, 0.75, 0.125], dtype=torch.float64)
+    sums = (2.0 ** 24 + 8.0) * w[:, None, None] * w[:, None] * w
+    lo = 4  # ghosted index of the stencil's first node
+    box = slice(lo, lo + len(w))
+    for op, a in zip(terms, arrays):
+        got = a.view()[box, box, box].double().cpu()
+        for d in range(got.shape[-1] if op != 4 else 0):
+            # (27 (2^24 + 8) / 64 and the like need one more rounding.)
+            assert torch.all((got[..., d] - sums).abs() <= sums * 2.0 ** -24), (op, d)
+
+
+@pytest.mark.parametrize("order", [1, 2, 3])
+def test_large_fp32_values_keep_the_fp64_window(ca, oracle, order):
+    """Values about 2^100 in crowded cells.  A node gets at most nine windows'
+    sums, each rounded to FP32 (2^-24), besides the roundings of the FP32
+    products and chains (2^-23): 12 * 2^-24.  One FP32 atomic a particle and
+    node would round thousands of times."""
+    c = Cloud(ca, oracle, 5, population=[200])
+    c.values[0] = np.float32(np.abs(c.values[0]) + 0.5).astype(np.float64) * 2.0 ** 100
+    own = c.mesh.owned_slices()
+    got, = c.p2g(ca, (0,), order, torch.float32)
+    ref = c.reference(oracle, 0, order, torch.float32)
+    assert rel_l2(got[own] * 2.0 ** -100, ref[own] * 2.0 ** -100) < 12 * 2.0 ** -24
