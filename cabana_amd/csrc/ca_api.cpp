@@ -866,6 +866,7 @@ bool make_tiles( TileKind kind, const MeshDev& m, int order, bool fp64,
     t.max_win_nodes = t.win[0] * t.win[1] * t.win[2];
     t.cap = sh.cap;
     t.sub = sh.sub;
+    t.thin = mean_ppc < SCATTER_THIN;
     t.bin_begin = bins->begin;
     // Window walk order: largest grid stride first.
     int perm[3] = { 0, 1, 2 };

@@ -353,6 +353,7 @@ struct TileArgs
     int32_t max_win_nodes;       // win[0] * win[1] * win[2]
     int32_t cap;                 // particles per part
     int32_t sub;                 // particles of a scatter's records in LDS
+    int32_t thin;                // fewer than SCATTER_THIN particles a cell
     int32_t grid;                // workgroups launched (a multiple of 8)
     int64_t bin_begin;           // particle index of cell offset 0
     // Particle at each binned position q (perm[q - bin_begin]) when the
@@ -395,6 +396,9 @@ constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
 //   8 (cubic): 0.26 0.29
 // (linear splines, 2, FP64: 0.51 0.54; the G2P adjoint at 3: 0.40 0.42).
 constexpr double SCATTER_SPARSE = 6.0;
+// Particles a cell below which the products of an FP32 group of up to four are
+// summed in two chains.
+constexpr double SCATTER_THIN = 4.0;
 constexpr int scatter_sub( int order, bool grad, int nslot, double mean_ppc )
 {
     return !grad || ( order > 1 && nslot > 1 && mean_ppc < SCATTER_SPARSE ) ? 16 : 32;

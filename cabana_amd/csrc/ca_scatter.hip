@@ -726,21 +726,30 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                     s = e;
                     while ( n > 0 )
                     {
-                        // FP32 products are summed over 8 particles at most for
-                        // a value-type tile and over 16 for a gradient-type
-                        // one, its three kinds apart, and the sums added in
-                        // FP64.  (Linear splines sum the three kinds in one
-                        // chain, but a lane's chain is of one particle a step,
-                        // 12 products at most.)  Relative L2 error of
-                        // momentum, 64^3 cells, quadratic, at 2, 8 and 16
-                        // particles a cell, e-8: 8.8 9.6 9.7; with chains of 16:
-                        // 8.8 9.9 10.5; the kernel before this one: 8.9 9.7
-                        // 10.3.  Each count of steps is code of its own, without
+                        // A chunk of one to four steps.  FP32 products are
+                        // summed over 8 particles at most for a value-type tile
+                        // and over 16 for a gradient-type one, its three kinds
+                        // apart, and the sums added in FP64.  (Linear splines
+                        // sum the three kinds in one chain, but a lane's chain
+                        // is of one particle a step, 12 products at most.)
+                        // KINDS is how the kinds of an FP32 gradient-type tile
+                        // are summed: 0 apart, 1 in one chain (groups of up to
+                        // four: 12 products), 2 in two chains added in FP64
+                        // (the same in thin clouds, where such groups are all
+                        // there is).  Relative L2 errors, 64^3 cells,
+                        // quadratic, of the kernel before this one and of this
+                        // one, e-8: momentum at 2, 8, 16 particles a cell 8.87
+                        // 9.71 10.3 and 8.84 9.60 9.70; stress divergence at 2,
+                        // 4, 8, 16: 9.44 10.0 10.6 11.3 and 9.23 10.0 10.5 11.1
+                        // (one chain at 2 a cell: 9.71; two cost the adjoint
+                        // 8 us of 98 there).
+                        // Each count of steps is code of its own, without
                         // branches, so that its operand reads are issued
                         // together: 1.87 -> 1.62 ms against a loop that read a
                         // step ahead.
-                        auto chunk = [&]( auto STEPS ) {
+                        auto chunk = [&]( auto STEPS, auto KINDS ) {
                             constexpr int NS = STEPS;
+                            constexpr int kinds = ORDER == 1 ? 1 : KINDS;
                             V4 D[NT][3];
                             Step<Real, ROW> st[NS];
                             static_for<NS>( [&]( auto C ) {
@@ -781,8 +790,8 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                 }
                                 static_for<NT>( [&]( auto T ) {
                                     constexpr int t = T;
-                                    constexpr int m1 = ORDER > 1 || !F32 ? 1 : 0;
-                                    constexpr int m2 = ORDER > 1 ? ( F32 ? 2 : 1 ) : ( F32 ? 0 : 2 );
+                                    constexpr int m1 = F32 && kinds > 0 ? 0 : 1;
+                                    constexpr int m2 = F32 ? ( kinds == 1 ? 0 : 2 ) : ( ORDER > 1 ? 1 : 2 );
                                     constexpr int dq = ORDER > 1 ? MF::QUAD : 0;
                                     constexpr int ds = ORDER > 1 ? MF::SLOT : 1;
                                     const Real* v = st[c].y + TL::val( t );
@@ -796,7 +805,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                             d = MF::mac( A, B, d );
                                     };
                                     if constexpr ( !TL::has_g( t ) )
-                                        mac( A1, wz * v[0], D[t][0] );
+                                        mac( A1, wz * v[0], D[t][F32 ? c / 2 : 0] );
                                     else
                                     {
                                         Real b1 = gz * h[2];
@@ -806,51 +815,43 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                                         mac( AQ, wz * h[dq], D[t][m1] );
                                         mac( AS, wz * h[ds], D[t][m2] );
                                     }
-                                    constexpr bool split = ( ORDER > 1 || !F32 ) && TL::has_g( t );
-                                    constexpr int CHAIN = F32 && !TL::has_g( t ) ? 2 : 4;
-                                    if constexpr ( c % CHAIN == CHAIN - 1 || c == NS - 1 )
-                                    {
-#pragma unroll
-                                        for ( int r = 0; r < NR; ++r )
-                                            if constexpr ( !F32 )
-                                            {
-                                                // (Chunks summed apart: one chain
-                                                // over all groups of a window
-                                                // measured up to 1.2 times the
-                                                // error.)
-                                                if constexpr ( !split )
-                                                    acc[t][r] += D[t][0][r];
-                                                else if constexpr ( ORDER == 1 )
-                                                    acc[t][r] += ( D[t][0][r] + D[t][1][r] ) + D[t][2][r];
-                                                else
-                                                    acc[t][r] += D[t][0][r] + D[t][1][r];
-                                            }
-                                            else if constexpr ( split && NS == 1 )
-                                                // Few particles: the roundings of
-                                                // the sum of the three kinds
-                                                // would be most of the error.
-                                                acc[t][r] +=
-                                                    ( (double)D[t][0][r] + (double)D[t][1][r] ) +
-                                                    (double)D[t][2][r];
-                                            else if constexpr ( split )
-                                                acc[t][r] += (double)( ( D[t][0][r] + D[t][1][r] ) +
-                                                                       D[t][2][r] );
-                                            else
-                                                acc[t][r] += (double)D[t][0][r];
-                                        if constexpr ( c < NS - 1 )
-                                            D[t][0] = V4{ 0, 0, 0, 0 };
-                                    }
                                 } );
                             } );
+                            static_for<NT>( [&]( auto T ) {
+                                constexpr int t = T;
+#pragma unroll
+                                for ( int r = 0; r < NR; ++r )
+                                    if constexpr ( !F32 && !TL::has_g( t ) )
+                                        // (Chunks summed apart: one chain over all
+                                        // groups of a window measured up to 1.2
+                                        // times the error.)
+                                        acc[t][r] += D[t][0][r];
+                                    else if constexpr ( !F32 && ORDER > 1 )
+                                        acc[t][r] += D[t][0][r] + D[t][1][r];
+                                    else if constexpr ( !F32 )
+                                        acc[t][r] += ( D[t][0][r] + D[t][1][r] ) + D[t][2][r];
+                                    else if constexpr ( TL::has_g( t ) && kinds == 0 )
+                                        acc[t][r] +=
+                                            (double)( ( D[t][0][r] + D[t][1][r] ) + D[t][2][r] );
+                                    else if constexpr ( TL::has_g( t ) && kinds == 2 )
+                                        acc[t][r] += (double)D[t][0][r] + (double)D[t][2][r];
+                                    else if constexpr ( !TL::has_g( t ) && NS > 2 )
+                                        acc[t][r] += (double)D[t][0][r] + (double)D[t][1][r];
+                                    else
+                                        acc[t][r] += (double)D[t][0][r];
+                            } );
                         };
+                        using std::integral_constant;
                         if ( MAX_STEPS == 4 && n > 12 )
-                            chunk( std::integral_constant<int, 4>{} );
+                            chunk( integral_constant<int, 4>{}, integral_constant<int, 0>{} );
                         else if ( MAX_STEPS == 4 && n > 8 )
-                            chunk( std::integral_constant<int, 3>{} );
+                            chunk( integral_constant<int, 3>{}, integral_constant<int, 0>{} );
                         else if ( n > 4 )
-                            chunk( std::integral_constant<int, 2>{} );
+                            chunk( integral_constant<int, 2>{}, integral_constant<int, 0>{} );
+                        else if ( F32 && TL::any_g() && ORDER > 1 && ta.thin )
+                            chunk( integral_constant<int, 1>{}, integral_constant<int, 2>{} );
                         else
-                            chunk( std::integral_constant<int, 1>{} );
+                            chunk( integral_constant<int, 1>{}, integral_constant<int, 1>{} );
                         n -= 4 * MAX_STEPS;
                         rp += 4 * MAX_STEPS * RS;
                     }
