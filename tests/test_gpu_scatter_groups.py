@@ -146,3 +146,36 @@ def test_large_fp32_values_keep_the_fp64_window(ca, oracle, order):
     got, = c.p2g(ca, (0,), order, torch.float32)
     ref = c.reference(oracle, 0, order, torch.float32)
     assert rel_l2(got[own] * 2.0 ** -100, ref[own] * 2.0 ** -100) < 12 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("moved", [0.05, 0.15, 0.6])
+@pytest.mark.parametrize("population", [POPULATION, SPARSE], ids=["dense", "sparse"])
+def test_positions_that_moved_since_the_binning(ca, oracle, order, dtype, moved, population):
+    """Batches whose cells are out of order are taken in cell order, and particles
+    of a quadratic spline up to half a cell out of their row keep its window: P2G
+    against the oracle, the G2P adjoint against the per-particle kernels."""
+    c = Cloud(ca, oracle, 57 + order, moved, population)
+    own = c.mesh.owned_slices()
+    for op, got in zip((0, 1, 4), c.p2g(ca, (0, 1, 4), order, dtype)):
+        assert rel_l2(got[own], c.reference(oracle, op, order, dtype)[own]) < TOL[dtype], op
+    rng = np.random.default_rng(3)
+    vbar = torch.tensor(rng.normal(size=(c.n, 3)), dtype=dtype, device="cuda")
+    lbar = torch.tensor(rng.normal(size=(c.n, 3, 3)), dtype=dtype, device="cuda")
+    u, ubar, uref = (ca.createArray("u", ca.createArrayLayout(c.lg, 3, ca.Node()), dtype=dtype)
+                     for _ in range(3))
+    halo = ca.createHalo(ca.NodeHaloPattern(), 1, u)
+    fs = [ca.createVectorValueG2P(vbar, 1.5), ca.createVectorGradientG2P(lbar, -0.5)]
+
+    def adjoint(out, bins):
+        ca.g2p_adjoint([u, u], halo, c.pts, c.n, ca.Spline(order), fs, [vbar, lbar], [out, out],
+                       None, bins=bins)
+
+    adjoint(ubar, c.bins)
+    ca.set_auto_binning(False)
+    try:
+        adjoint(uref, None)
+    finally:
+        ca.set_auto_binning(True)
+    assert rel_l2(ubar.view().cpu().numpy()[own], uref.view().cpu().numpy()[own]) < TOL[dtype]
