@@ -1,6 +1,7 @@
 // C-ABI layer: descriptor validation, plan selection and kernel dispatch.
 #include "ca_internal.hpp"
 
+#include <algorithm>
 #include <rocprofiler-sdk-roctx/roctx.h>
 
 #include <atomic>
@@ -792,22 +793,34 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
         }
         return found;
     }
-    // Scatters: the brick with the most cells per window node (fewest grid
-    // atomics per cell) whose LDS lets a full set of workgroups run on a CU,
-    // among those that give every CU two bricks: MPM P2G of 32^3 cells x 8,
-    // FP32, takes 53 us with at least 1024 bricks (whose windows add more nodes
-    // to the grid, each rounded to FP32), 43 us with 512 and 48 us with 256.
+    // Scatters: the shape of least estimated time, (particles + node_cost *
+    // window nodes) of a part times the rounds its launch takes (slots: the
+    // workgroups that run at once), the last of which is partly filled.  Fitted to
+    // the 13 shapes of 31 meshes, P2G and G2P adjoint: the shape taken is 0.7 % off
+    // the fastest in the mean and 10 % at most, where the largest brick that leaves
+    // 512 of them lost up to a third (the FP64 G2P adjoint of 64^3 x 16, quadratic:
+    // 301 us with 4 x 4 x 8 cells, 317 with 6 x 6 x 8, 443 with 8 x 8 x 8).  A part
+    // is a whole brick, or an equal share of it of 1024 particles or more where
+    // there are few bricks.
+    // In FP32 every part's sums are rounded as they are added to the grid (and
+    // the longer chains of dense cells have their own error), so a part has 300
+    // particles and 50 a cell at least (1000 at most), or the largest brick: with
+    // 2 x 2 x 8 cells for 20 x 24 x 18 x 2, momentum has an error of 9.6e-8, with
+    // 5 x 5 x 8 8.8e-8 (the kernel before the matrix cores: 8.8e-8).
     // Above 2^20 bricks, where the part table itself is large, two workgroups
     // per CU.
     const int extra = ( order == 1 ) ? 1 : 3;
     const int c = scatter_cells_k( order );
     const int waves = scatter_waves( fp64, scatter_grad( vals ) );
     const int sub = scatter_sub( order, scatter_grad( vals ), nslot, mean_ppc );
+    const double node_cost = order == 1 ? 8.0 : 3.0;
     bool found = false;
     double best_bricks = 0.0;
     for ( int w = waves; w >= 2 && ( !found || best_bricks > 1048576.0 ); w = w > 2 ? 2 : 1 )
     {
-        double best = -1.0;
+        const double slots = 256.0 * w;
+        double best = 0.0, best_held = 0.0;
+        bool first = true;
         for ( int a = 2; a <= 8; ++a )
             for ( int b = a; b <= a + 1 && b <= 8; ++b )
             {
@@ -816,17 +829,31 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
                      (size_t)scatter_lds( w ) )
                     continue;
                 const double bricks = bricks_of( sh );
-                const double share = (double)( a * b ) / ( ( a + extra ) * ( b + extra ) );
-                const double score = share * ( bricks < 512.0 ? bricks / 512.0 : 1.0 );
-                if ( score <= best )
-                    continue;
-                best = score;
-                best_bricks = bricks;
-                found = true;
-                double cap = 1.25 * mean_ppc * a * b * c;
-                cap = cap < 1024 ? 1024 : ( cap > 8192 ? 8192 : cap );
-                sh.cap = ( (int)cap + 63 ) / 64 * 64;
-                out = sh;
+                const double nodes = (double)( a + extra ) * ( b + extra ) * ( c + extra );
+                const double brick = mean_ppc * a * b * c;
+                for ( double cuts = 1.0; cuts == 1.0 || ( brick / cuts >= 1024.0 &&
+                                                          bricks * cuts <= 2.0 * slots );
+                      cuts *= 2.0 )
+                {
+                    const double rounds = std::max( bricks * cuts / slots, 1.0 );
+                    const double time = ( brick / cuts + node_cost * nodes ) *
+                                        ( 0.4 * rounds + 0.6 * std::ceil( rounds ) + 0.3 );
+                    // Particles a part holds, as far as the FP32 rule asks for them.
+                    const double held =
+                        fp64 ? 0.0
+                             : std::min( { brick / cuts, 300.0 + 50.0 * mean_ppc, 1000.0 } );
+                    if ( !first && ( held < best_held || ( held == best_held && time >= best ) ) )
+                        continue;
+                    first = false;
+                    best = time;
+                    best_held = held;
+                    best_bricks = bricks;
+                    found = true;
+                    double cap = 1.25 * brick / cuts;
+                    cap = cap < 1024 ? 1024 : ( cap > ( 1 << 20 ) ? ( 1 << 20 ) : cap );
+                    sh.cap = ( (int)cap + 63 ) / 64 * 64;
+                    out = sh;
+                }
             }
     }
     return found;

@@ -505,9 +505,10 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
     // windows of the linear spline are three cells apart and do not slide.)
     constexpr bool SLIDE = ORDER != 1;
     // Steps of a chunk at most: the fused passes of sparse particles (records of
-    // 16) seldom have more than eight in a group, and chunks of four cost them
-    // 32 spilled registers.
-    constexpr int MAX_STEPS = SUB == 16 && TL::any_g() ? 2 : 4;
+    // 16) seldom have more than eight in a group, and chunks of four cost them,
+    // and the FP32 P2G of linear splines, 30 to 40 spilled registers.
+    constexpr int MAX_STEPS =
+        TL::any_g() && ( SUB == 16 || ( ORDER == 1 && F32 && NT == 2 ) ) ? 2 : 4;
     extern __shared__ __align__( 16 ) unsigned char smem[];
 
     // LDS: the FP64 node window (one block per tile, [node][dof]), the waves'
