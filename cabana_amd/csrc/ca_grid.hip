@@ -1181,14 +1181,26 @@ __global__ __launch_bounds__( BLOCK ) void compact_index_kernel( const int32_t* 
         idx[rank[p]] = p;
 }
 
-// The same keys counted as they are formed: rank[p] is the particle's arrival
+// Owned-cell keys counted as they are formed: rank[p] is the particle's arrival
 // number in its cell.  Lanes of a wave with equal keys next to each other
-// (particles near cell order) share one atomic.
-__global__ __launch_bounds__( BLOCK ) void auto_bin_rank_kernel( PFieldDev pos, int64_t n, MeshDev m,
-                                                                 int32_t* keys, int32_t* counts,
-                                                                 int32_t* rank )
+// (particles near cell order) count together, then the workgroup's equal keys in
+// an LDS hash table, so that a cell takes one global atomic a workgroup however
+// crowded it is: one atomic a run of lanes reaches 170 M/s on one counter, and
+// 10^6 particles of two cells in random order took 2.97 ms.
+constexpr int RANK_BLOCK = 1024;
+constexpr int RANK_TABLE = 2 * RANK_BLOCK; // half of it free: a probe always ends
+__global__ __launch_bounds__( RANK_BLOCK ) void auto_bin_rank_kernel( PFieldDev pos, int64_t n,
+                                                                      MeshDev m, int32_t* keys,
+                                                                      int32_t* counts, int32_t* rank )
 {
-    const int64_t p = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    __shared__ int tkey[RANK_TABLE];   // key, -1 free
+    __shared__ int tcount[RANK_TABLE]; // particles of the key, then its first rank
+    for ( int e = threadIdx.x; e < RANK_TABLE; e += RANK_BLOCK )
+    {
+        tkey[e] = -1;
+        tcount[e] = 0;
+    }
+    const int64_t p = (int64_t)blockIdx.x * RANK_BLOCK + threadIdx.x;
     const bool ok = p < n;
     const int key = ok ? owned_cell( pos, p, m ) : -1;
     const int lane = threadIdx.x & 63;
@@ -1198,16 +1210,33 @@ __global__ __launch_bounds__( BLOCK ) void auto_bin_rank_kernel( PFieldDev pos, 
     const int lead = 63 - __clzll( (long long)( starts & ( ~0ull >> ( 63 - lane ) ) ) );
     const uint64_t after = lane == 63 ? 0ull : starts >> ( lane + 1 );
     const int end = after ? lane + 1 + __builtin_ctzll( after ) : 64;
-    int base = 0;
+    __syncthreads();
+    int slot = 0, first = 0;
     if ( ok && lane == lead )
-        base = atomicAdd( counts + key, end - lead );
-    base = __shfl( base, lead, 64 );
+    {
+        slot = (int)( (uint32_t)key * 2654435761u >> 21 );
+        int held = atomicCAS( &tkey[slot], -1, key );
+        while ( held != -1 && held != key )
+        {
+            slot = ( slot + 1 ) & ( RANK_TABLE - 1 );
+            held = atomicCAS( &tkey[slot], -1, key );
+        }
+        first = atomicAdd( &tcount[slot], end - lead );
+    }
+    __syncthreads();
+    for ( int e = threadIdx.x; e < RANK_TABLE; e += RANK_BLOCK )
+        if ( tkey[e] >= 0 )
+            tcount[e] = atomicAdd( counts + tkey[e], tcount[e] );
+    __syncthreads();
+    slot = __shfl( slot, lead, 64 );
+    first = __shfl( first, lead, 64 );
     if ( ok )
     {
         keys[p] = key;
-        rank[p] = base + lane - lead;
+        rank[p] = tcount[slot] + first + lane - lead;
     }
 }
+static_assert( RANK_TABLE == 1 << 11, "the hash keeps 11 bits" );
 
 __global__ __launch_bounds__( BLOCK ) void auto_bin_place_kernel( const int32_t* keys,
                                                                   const int32_t* rank, int64_t n,
@@ -1853,8 +1882,9 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
     if ( e != hipSuccess )
         return e;
     L.before( "auto_bin_keys", s );
-    hipLaunchKernelGGL( auto_bin_rank_kernel, blocks_for( n ), dim3( BLOCK ), 0, s, pos, n, m, keys,
-                        counts, rank );
+    hipLaunchKernelGGL( auto_bin_rank_kernel,
+                        dim3( (unsigned)( ( n + RANK_BLOCK - 1 ) / RANK_BLOCK ) ),
+                        dim3( RANK_BLOCK ), 0, s, pos, n, m, keys, counts, rank );
     L.after( "auto_bin_keys", s );
     e = launch_exclusive_scan( L, counts, offsets, ncell, block_sums, nblock_cap, s );
     if ( e != hipSuccess )
@@ -1866,12 +1896,16 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
     return hipGetLastError();
 }
 
-// Counting needs four launches against the sort's three a pass, but its
-// atomics reach about 24 G/s on random particles.  P2G and G2P of mass and
-// momentum, unbinned, counting and sorting: 262144 particles on 32^3 cells 134
-// and 177 us, 1.06 M on 51^3 cells 336 and 350, 1.56 M on 58^3 cells 471 and
-// 446, 2.1 M on 64^3 cells 577 and 497.  Few cells would contend for their
-// counters.
+// Counting takes four launches (six above 65536 cells, where the scan takes
+// three) against the sort's three a pass.  P2G and G2P of mass and momentum,
+// unbinned, counting and sorting, uniform clouds in random order: 262144 particles
+// on 32^3 cells 134 and 177 us, 1.06 M on 51^3 cells 336 and 350, 1.56 M on 58^3
+// cells 471 and 446, 2.1 M on 64^3 cells 577 and 497.  Crowded clouds gain more:
+// G2P of 10^6 particles in two cells of 64^3 94 and 218 us, in a Gaussian blob of
+// 1.5 cells 171 and 237.  On meshes of few cells the sort has fewer passes, and
+// the transfers read its order faster (ascending within a cell): G2P of 10^6 on
+// 24^3 (72 a cell) 142 and 125 us, on 16^3 164 and 127, on 8^3 420 and 200; on
+// 32^3 (31 a cell) counting is the faster one, 143 and 279 (one more pass).
 bool auto_bin_counts( int64_t n, int64_t ncell )
 {
     return n > RS_SMALL_MAX && n <= ( 1 << 20 ) + ( 1 << 17 ) && n / ncell <= 64;

@@ -77,3 +77,44 @@ def test_calls_without_a_binning(ca, oracle, n, cells, order, cell_order):
     ref = np.zeros((n, 3))
     oracle.g2p(mesh, order, 1, 1.0, u, pts, ref)
     assert rel_l2(out.cpu().numpy(), ref) < TOL[torch.float64]
+
+
+def crowd(kind, n, cells, rng):
+    """Positions in random order: everywhere, in a few cells, in one, in a blob."""
+    if kind == "uniform":
+        return rng.uniform(0.0, cells, size=(n, 3))
+    if kind == "blob":
+        return np.clip(cells / 2 + 1.5 * rng.normal(size=(n, 3)), 0.0, cells - 1e-9)
+    few = rng.integers(0, cells, size=(1 if kind == "one" else 3, 3))
+    return few[rng.integers(0, len(few), size=n)] + rng.uniform(0.0, 1.0, size=(n, 3))
+
+
+# The counting build: a crowded cell's particles share one counter, above 65536
+# cells (41^3) its scan takes three launches, and it ends at 2^20 + 2^17 particles.
+@pytest.mark.parametrize("kind", ["uniform", "few", "one", "blob"])
+@pytest.mark.parametrize("n,cells", [(16385, 40), (70001, 41), ((1 << 20) + (1 << 17), 41),
+                                     ((1 << 20) + (1 << 17) + 1, 41)])
+def test_counting_build_of_crowded_clouds(ca, oracle, kind, n, cells):
+    rng = np.random.default_rng(n % 1000 + cells)
+    pts = crowd(kind, n, cells, rng)
+    gm = ca.createUniformGlobalMesh([0.0] * 3, [float(cells)] * 3, 1.0)
+    lg = ca.createLocalGrid(ca.createGlobalGrid(gm, [True] * 3), 1)
+    mesh = oracle.OMesh([0.0] * 3, [float(cells)] * 3, 1.0, halo=1)
+    rho = ca.createArray("rho", ca.createArrayLayout(lg, 1, ca.Node()))
+    halo = ca.createHalo(ca.NodeHaloPattern(), 1, rho)
+    mass = rng.uniform(0.5, 1.5, size=n)
+    x = torch.tensor(pts, device="cuda")
+    ca.p2g(ca.createScalarValueP2G(torch.tensor(mass, device="cuda"), 1.0), x, n, ca.Spline(1),
+           halo, rho)
+    ref = mesh.grid(1)
+    oracle.p2g(mesh, 1, 0, 1.0, pts, mass[:, None], ref)
+    own = mesh.owned_slices()
+    assert rel_l2(rho.view().cpu().numpy()[own], ref[own]) < TOL[torch.float64]
+    u = rng.normal(size=tuple(mesh.num_node) + (1,))
+    grid = ca.createArray("u", ca.createArrayLayout(lg, 1, ca.Node()))
+    grid.view().copy_(torch.tensor(u))
+    out = torch.zeros(n, dtype=torch.float64, device="cuda")
+    ca.g2p(grid, halo, x, n, ca.Spline(1), ca.createScalarValueG2P(out, 1.0))
+    ref = np.zeros((n, 1))
+    oracle.g2p(mesh, 1, 0, 1.0, u, pts, ref)
+    assert rel_l2(out.cpu().numpy()[:, None], ref) < TOL[torch.float64]
