@@ -812,7 +812,7 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
     const int extra = ( order == 1 ) ? 1 : 3;
     const int c = scatter_cells_k( order );
     const int waves = scatter_waves( fp64, scatter_grad( vals ) );
-    const int sub = scatter_sub( order, scatter_grad( vals ), nslot, mean_ppc );
+    const int sub = scatter_sub( fp64, order, scatter_grad( vals ), nslot, mean_ppc );
     const double node_cost = order == 1 ? 8.0 : 3.0;
     bool found = false;
     double best_bricks = 0.0;

@@ -389,19 +389,20 @@ constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
 // leave the window more room (and cost a wave per SIMD with value terms if
 // they were 64), 32 break fewer runs of one cell apart.  Value terms take 16:
 // mass and momentum of 8.4 M clustered particles 0.46 ms against 0.50 ms.
-// Gradient terms take 32, the fused MPM P2G below SCATTER_SPARSE particles a
-// cell 16, in ms with 32 and with 16 (quadratic unless said):
-//   FP32, particles a cell:  2: 0.91 0.85   6: 0.48 0.44   16: 1.52 1.67
-//   FP64:  2: 1.28 1.16   3 (cubic): 0.72 0.61   4: 0.94 0.88   16: 1.24 1.38
-//   8 (cubic): 0.26 0.29
-// (linear splines, 2, FP64: 0.51 0.54; the G2P adjoint at 3: 0.40 0.42).
-constexpr double SCATTER_SPARSE = 6.0;
+// Gradient terms take 32, the fused MPM P2G below scatter_sparse particles a cell
+// 16.  us with 32 and with 16, quadratic, 96^3 cells (80^3 from 10 a cell on):
+//   a cell    2        3        4        5        6        7        8        10
+//   FP32  397 386  483 422  439 441  498 504  463 479  491 519  495 527  338 347
+//   FP64  570 573  714 601  652 598  769 628  713 681  818 734  792 795  527 554
+// (cubic splines and clustered clouds the same; linear splines, 2, FP64: 0.51
+// 0.54 ms; the G2P adjoint at 3: 0.40 0.42 ms).
+constexpr double scatter_sparse( bool fp64 ) { return fp64 ? 8.0 : 4.0; }
 // Particles a cell below which the products of an FP32 group of up to four are
 // summed in two chains.
 constexpr double SCATTER_THIN = 4.0;
-constexpr int scatter_sub( int order, bool grad, int nslot, double mean_ppc )
+constexpr int scatter_sub( bool fp64, int order, bool grad, int nslot, double mean_ppc )
 {
-    return !grad || ( order > 1 && nslot > 1 && mean_ppc < SCATTER_SPARSE ) ? 16 : 32;
+    return !grad || ( order > 1 && nslot > 1 && mean_ppc < scatter_sparse( fp64 ) ) ? 16 : 32;
 }
 // Cells of a scatter brick along k, a compile-time stride of the LDS window
 // (linear splines: groups of three cells).

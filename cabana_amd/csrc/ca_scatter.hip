@@ -991,7 +991,7 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
 template <int F>
 constexpr int single_sub()
 {
-    return scatter_sub( ORDER, Tiles<false, F>::any_g(), 1, 0.0 );
+    return scatter_sub( false, ORDER, Tiles<false, F>::any_g(), 1, 0.0 );
 }
 
 template <class Real, bool CONTIG>

@@ -16,8 +16,10 @@ pytestmark = pytest.mark.gpu
 
 POPULATION = [0, 1, 2, 3, 4, 5, 7, 8, 9, 0, 12, 13, 15, 16, 17, 20, 31, 32, 33, 48, 63, 64, 65,
               0, 0, 130]
-# Below 6 a cell, where the fused MPM P2G keeps the records of 16 particles.
+# 5.1 a cell, where the fused FP64 MPM P2G keeps the records of 16 particles; 3.0,
+# where the FP32 one does too and sums groups of up to four in two chains.
 SPARSE = [0, 1, 2, 3, 4, 0, 0, 16, 17, 0, 0, 1, 33, 0, 0, 5]
+THIN = [0, 1, 2, 3, 4, 0, 0, 16, 17, 0, 0, 1, 0, 0, 0, 4]
 CELLS = (5, 7, 19)
 CELL = 0.5
 LOW = np.array([0.25, -1.0, 2.0])
@@ -179,3 +181,15 @@ def test_positions_that_moved_since_the_binning(ca, oracle, order, dtype, moved,
     finally:
         ca.set_auto_binning(True)
     assert rel_l2(ubar.view().cpu().numpy()[own], uref.view().cpu().numpy()[own]) < TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("order", [1, 2, 3])
+@pytest.mark.parametrize("moved", [0.0, 0.15])
+def test_thin_clouds(ca, oracle, order, dtype, moved):
+    c = Cloud(ca, oracle, 91 + order, moved, THIN)
+    own = c.mesh.owned_slices()
+    for ops in SETS:
+        for op, got in zip(ops, c.p2g(ca, ops, order, dtype)):
+            ref = c.reference(oracle, op, order, dtype)
+            assert rel_l2(got[own], ref[own]) < TOL[dtype], (ops, op)
