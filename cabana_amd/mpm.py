@@ -103,8 +103,11 @@ def explicit_step(box, x, v, m, dt=0.1, body_force=(0.0, 0.0, -1e-3), resort=Tru
         record.append((mass.detach(), mom.detach()))
     # From pinned memory: a copy from pageable memory makes the host wait for
     # the sort and the P2G before it can launch the rest of the step.
-    f = torch.tensor(body_force, dtype=mom.dtype, device="cpu", pin_memory=mom.is_cuda)
-    f = f.to(mom.device, non_blocking=True)
+    if isinstance(body_force, torch.Tensor):
+        f = body_force.detach().to(dtype=mom.dtype, device=mom.device)
+    else:
+        f = torch.tensor(body_force, dtype=mom.dtype, device="cpu", pin_memory=mom.is_cuda)
+        f = f.to(mom.device, non_blocking=True)
     u = (mom + (dt * f) * mass) / (mass + mass_floor)
     vn, grad_v = AG.g2p(x, [u, u], lg, ["VectorValue", "VectorGradient"], order=2, bins=bins)
     xn = periodic_wrap(box, x + dt * vn.to(x.dtype))

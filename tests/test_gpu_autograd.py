@@ -257,3 +257,28 @@ def test_loop_gradient_fd(ca):
                     worst = max(worst, err)
     print("loop gradient vs FD: worst relative error %.3e" % worst)
     assert worst <= 1e-6
+
+
+@pytest.mark.parametrize("kind", ["tuple", "device", "host"])
+def test_body_force_of_an_mpm_step(ca, kind):
+    """A body force in any form gives the same step; one that is on the device
+    already, or a tuple, does not make the host wait for the stream."""
+    from cabana_amd import mpm
+
+    box = mpm.PeriodicBox(6)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.rand(500, 3, dtype=torch.float64, device="cuda", generator=g) * 6.0
+    v = torch.randn(500, 3, dtype=torch.float64, device="cuda", generator=g)
+    m = torch.rand(500, dtype=torch.float64, device="cuda", generator=g) + 0.5
+    force = (0.5, -0.25, 2.0)
+    ref = mpm.explicit_step(box, x, v, m, body_force=force)
+    if kind != "tuple":
+        force = torch.tensor(force, dtype=torch.float64, device="cuda" if kind == "device" else "cpu")
+    torch.cuda.synchronize()
+    torch.cuda.set_sync_debug_mode("error" if kind != "host" else "default")
+    try:
+        got = mpm.explicit_step(box, x, v, m, body_force=force)
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    for a, b in zip(got, ref):
+        assert (a - b).norm() <= 1e-12 * b.norm()
