@@ -307,18 +307,30 @@ def test_fused_mpm_transfer(ca, oracle, order, dtype, sorted_bins):
 
 @pytest.mark.parametrize("order", [1, 2, 3])
 def test_fused_mpm_many_parts_per_workgroup(ca, oracle, order, monkeypatch):
-    """Eight workgroups for ~1600 parts (16 particles per cell): every
-    workgroup walks ~200 parts, so the scatter's part-table refills and
-    run-table double buffers cycle many times.  P2G (mass, momentum, stress
-    divergence) against the oracle, FP32-mixed."""
+    """Eight workgroups for a cloud whose parts number thousands, most of them
+    several to a brick: a cluster of 1.4 M particles in a mesh of a million
+    cells.  A part holds at most 1.25 times what a brick (8 x 8 x 9 cells or
+    fewer) has in the mean, and 1024 if that is less, so every workgroup walks
+    more than 150 parts and reuses its window and run table as often.  P2G
+    (mass, momentum, stress divergence) against the oracle, FP32-mixed."""
     monkeypatch.setenv("CABANA_AMD_MAX_TILE_GROUPS", "8")
     dtype = torch.float32
-    c = Case(ca, oracle, num_cell=(36, 36, 34), n=700000, seed=77 + order)
+    cells, n = (128, 128, 64), 1500000
+    part = max(1024.0, 1.25 * n / np.prod(cells) * 8 * 8 * 9)
+    assert n / part / 8 > 150
+    low = np.array([0.25, -1.0, 2.0])
+    c = Case(ca, oracle, num_cell=cells, n=n, seed=77 + order, low=low)
+    size = 0.25 * np.array(cells)
+    dense = n - n // 15
+    c.pts_np[:dense] = low + np.mod(
+        size / 2 + c.rng.normal(scale=[1.5, 0.75, 1.0], size=(dense, 3)), size)
+    c.pts = torch.tensor(c.pts_np, device="cuda")
     m, q, sig = mpm_fields(c, dtype)
     gm = c.lg.globalGrid().globalMesh()
     lo = [gm.lowCorner(d) for d in range(3)]
     hi = [gm.highCorner(d) for d in range(3)]
     lcl = ca.createLinkedCellList(c.pts, [gm.cellSize(d) for d in range(3)], lo, hi)
+    assert [lcl.numBin(d) for d in range(3)] == list(cells)
     perm = lcl.permutes.cpu().numpy()
     pts = c.pts[lcl.permutes].contiguous()
     pts_np = c.pts_np[perm]
@@ -446,8 +458,9 @@ def test_invalid_arguments_raise(ca, oracle):
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("order", [1, 2, 3])
 def test_dense_cells_multiple_batches(ca, oracle, order, dtype):
-    """~200 particles per cell in a cluster: bricks exceed the per-batch sort
-    capacity and base cells are flushed in several batches."""
+    """~280 particles per cell in the mean, thousands in the middle of a cluster:
+    one cell fills many batches of 64 and chunks of 16, and a brick several
+    parts."""
     c = Case(ca, oracle, num_cell=(6, 6, 6), cell=0.5, n=1, seed=17)
     rng = np.random.default_rng(17)
     gm = c.lg.globalGrid().globalMesh()
