@@ -709,9 +709,7 @@ enum TileKind
     TILE_SCATTER = 1
 };
 
-constexpr int TILE_BLOCK = 256;
-
-// Workgroups of a tiled launch (a multiple of 8, one range per XCD): 4096 by
+// Workgroups of a tiled launch (a multiple of 8, as many on each XCD): 4096 by
 // default; CABANA_AMD_MAX_TILE_GROUPS lowers it (tests use it to give every
 // workgroup many parts).
 int64_t max_tile_groups()
@@ -1720,12 +1718,6 @@ extern "C" cabana_amd_status cabana_amd_g2p(
 // ---------------------------------------------------------------------------
 // G2P followed by P2G in one call
 // ---------------------------------------------------------------------------
-
-namespace
-{
-// Bytes from a grid's first element to one past its last.
-
-} // namespace
 
 extern "C" cabana_amd_status cabana_amd_g2p2g(
     cabana_amd_context* ctx, const cabana_amd_mesh* mesh, int32_t order,

@@ -226,8 +226,8 @@ __device__ __forceinline__ int64_t locate_cell( const CartGridDev& g,
 }
 
 // Bin key of every particle in [begin, end): its cardinal cell, or bad_key
-// (one past the last cell) when the particle lies outside the grid.  No
-// per-cell counters are touched here: the counts come out of the sort.
+// (one past the last cell) when the particle lies outside the grid.  The
+// cells' counts come out of the sorted keys.
 struct CartKey
 {
     PFieldDev pos;
@@ -993,10 +993,9 @@ __global__ __launch_bounds__( BLOCK ) void permute_put_words_kernel(
     dst[( begin + (int64_t)i ) * row_words + j] = scratch[w];
 }
 
-// Part table of a brick tiling.  One thread per brick counts the brick's
-// particles through the cell offsets of its cell runs and the number of
-// parts of at most t.cap particles (an empty brick has none).
-// BRICK_LANES lanes sum the cell rows of a brick.
+// Part table of a brick tiling: the brick's particles, counted through the cell
+// offsets of its cell rows by BRICK_LANES lanes, make parts of at most t.cap
+// particles (an empty brick has none).
 constexpr int BRICK_LANES = 8;
 // Particles of brick b, to every lane of its group of BRICK_LANES.
 __device__ __forceinline__ int64_t brick_count( const TileArgs& t, int3 nc, int b, int sub )

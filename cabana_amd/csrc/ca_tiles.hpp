@@ -33,7 +33,6 @@ constexpr int BLOCK = 256;
 // Stencil base node of a particle in cell c (ghosted node index):
 // c + halo + BASE_SHIFT + {0, 1 if ORDER == 2}.
 constexpr int BASE_SHIFT = ( ORDER == 1 ) ? 0 : -1;
-constexpr int BASE_SPREAD = ( ORDER == 2 ) ? 1 : 0;
 template <int... FORMS>
 struct FormList
 {
@@ -51,10 +50,6 @@ constexpr int np_of( int form )
                ? 1
                : ( ( form == FORM_VV || form == FORM_VD ) ? 3 : 9 );
 }
-// LDS dof stride of a staged grid: 3-dof nodes are padded to 4 so one
-// 128-bit LDS read fetches a node.
-constexpr int ngp_of( int form ) { return ng_of( form ) == 1 ? 1 : 4; }
-
 __device__ __forceinline__ size_t align16( size_t b )
 {
     return ( b + 15 ) & ~(size_t)15;
@@ -150,24 +145,6 @@ __device__ __forceinline__ int setup_runs( const TileArgs& ta,
     }
     __syncthreads();
     return run_pre[nruns];
-}
-
-// Particle index of flattened brick position v (binary search of the runs).
-__device__ __forceinline__ int64_t run_particle( const TileArgs& ta,
-                                                 const int64_t* run_start,
-                                                 const int* run_pre, int nruns,
-                                                 int v )
-{
-    int lo = 0, hi = nruns - 1;
-    while ( lo < hi )
-    {
-        const int mid = ( lo + hi + 1 ) >> 1;
-        if ( run_pre[mid] <= v )
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return ta.particle( ta.bin_begin + run_start[lo] + ( v - run_pre[lo] ) );
 }
 
 // Run containing flattened brick position v (binary search).
