@@ -723,17 +723,17 @@ __global__ __launch_bounds__( BLOCK ) void lcl_bounds_kernel(
 }
 
 // The whole build of up to RS_SMALL_BLOCK * ITEMS particles by one workgroup:
-// the keys are formed in registers; every
-// pass stays in LDS (keys, 16-bit indices, per-wave digit counts), with the
-// ranks of radix_scatter_kernel; then the permutation and, for up to
-// RS_SMALL_CELLS bins, counts and offsets by binary search of the keys in LDS.
-// At these sizes the launches of the tiled sort (three a pass) and of the
-// bounds are what a build costs: 4096 particles in 512 cells take 13 us
-// against 100 us.
+// the keys are formed in registers; every pass stays in LDS (keys, 16-bit
+// indices, per-wave digit counts), with the ranks of radix_scatter_kernel; then
+// the permutation and, for up to RS_SMALL_CELLS bins, counts and offsets by binary
+// search of the keys in LDS.  At these sizes the launches of the tiled sort (three
+// a pass) and of the bounds are what a build costs: 4096 particles in 32^3 cells
+// take 55 us against 100, 8192 (eight keys a thread) 66 against 102; 16384 (sixteen)
+// took 159 against 105 and go to the tiled sort.
 constexpr int RS_SMALL_BLOCK = 1024;
 constexpr int RS_SMALL_WAVES = RS_SMALL_BLOCK / 64;
 constexpr int64_t RS_SMALL_CELLS = 16384;
-constexpr int64_t RS_SMALL_MAX = RS_SMALL_BLOCK * 16;
+constexpr int64_t RS_SMALL_MAX = RS_SMALL_BLOCK * 8;
 
 template <int ITEMS>
 constexpr size_t rs_small_lds()
@@ -1460,12 +1460,12 @@ hipError_t bin_sort( Launcher& L, const char* name, const Key& key, int64_t begi
     const int passes = lcl_sort_passes( key_bits, &dbits );
     if ( n <= RS_SMALL_MAX )
     {
-        // One workgroup (four or sixteen keys a thread).
+        // One workgroup (four or eight keys a thread).
         const hipError_t e =
             n <= 4 * RS_SMALL_BLOCK
                 ? launch_sort_small<4>( L, name, key, begin, n, passes, dbits, permutes, w.keys_b, ncell,
                                         counts, offsets, s )
-                : launch_sort_small<16>( L, name, key, begin, n, passes, dbits, permutes, w.keys_b, ncell,
+                : launch_sort_small<8>( L, name, key, begin, n, passes, dbits, permutes, w.keys_b, ncell,
                                          counts, offsets, s );
         if ( e != hipSuccess || ncell <= RS_SMALL_CELLS )
             return e;
@@ -1896,7 +1896,9 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
 }
 
 // Counting takes four launches (six above 65536 cells, where the scan takes
-// three) against the sort's three a pass.  P2G and G2P of mass and momentum,
+// three) against the sort's three a pass, or its one up to 8192 particles: G2P of
+// 5000 on 32^3 cells takes 48 us counting and 50 sorting, of 8192 48 and 54, of
+// 4096 (sorting) 45.  P2G and G2P of mass and momentum,
 // unbinned, counting and sorting, uniform clouds in random order: 262144 particles
 // on 32^3 cells 134 and 177 us, 1.06 M on 51^3 cells 336 and 350, 1.56 M on 58^3
 // cells 471 and 446, 2.1 M on 64^3 cells 577 and 497.  Crowded clouds gain more:
@@ -1907,7 +1909,7 @@ hipError_t launch_auto_bin_count( Launcher& L, const PFieldDev& pos, int64_t n, 
 // 32^3 (31 a cell) counting is the faster one, 143 and 279 (one more pass).
 bool auto_bin_counts( int64_t n, int64_t ncell )
 {
-    return n > RS_SMALL_MAX && n <= ( 1 << 20 ) + ( 1 << 17 ) && n / ncell <= 64;
+    return n > 4096 && n <= ( 1 << 20 ) + ( 1 << 17 ) && n / ncell <= 64;
 }
 
 } // namespace cabana_amd
