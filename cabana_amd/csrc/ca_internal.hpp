@@ -392,11 +392,12 @@ constexpr int scatter_lds( int waves ) { return 160 * 1024 / waves - 512; }
 // Gradient terms take 32, the fused MPM P2G below scatter_sparse particles a cell
 // 16.  us with 32 and with 16, quadratic, 96^3 cells (80^3 from 10 a cell on):
 //   a cell    2        3        4        5        6        7        8        10
-//   FP32  397 386  483 422  439 441  498 504  463 479  491 519  495 527  338 347
-//   FP64  570 573  714 601  652 598  769 628  713 681  818 734  792 795  527 554
-// (cubic splines and clustered clouds the same; linear splines, 2, FP64: 0.51
-// 0.54 ms; the G2P adjoint at 3: 0.40 0.42 ms).
-constexpr double scatter_sparse( bool fp64 ) { return fp64 ? 8.0 : 4.0; }
+//   FP32  435 363  472 424  462 463  481 450  471 475  477 492  485 509  328 341
+//   FP64  634 517  680 551  703 566  754 614  755 666  785 722  795 783  510 543
+// (cubic splines the same; clustered clouds, FP32 at 4 and 8: 418 420  522 549,
+// FP64: 590 571  802 875; linear splines, 2, FP64: 0.51 0.54 ms; the G2P adjoint
+// at 3: 0.40 0.42 ms).
+constexpr double scatter_sparse( bool fp64 ) { return fp64 ? 8.0 : 6.0; }
 // Particles a cell below which the products of an FP32 group of up to four are
 // summed in two chains.
 constexpr double SCATTER_THIN = 4.0;

@@ -570,8 +570,9 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
         [[maybe_unused]] const float rnj = 1.0f / (float)nj;
         const int pbeg = tg.part * ta.cap;
         const int pend = min( run_pre[nruns], pbeg + ta.cap );
-        // The wave's share: a contiguous range of whole batches.
-        const int per = ( ( pend - pbeg + NWAVE * 64 - 1 ) / ( NWAVE * 64 ) ) * 64;
+        // The wave's share: a contiguous range, equal to 16 particles (equal to a
+        // batch, one wave of a part of a few batches had little or nothing).
+        const int per = ( ( pend - pbeg + NWAVE * 16 - 1 ) / ( NWAVE * 16 ) ) * 16;
         const int v0 = __builtin_amdgcn_readfirstlane( pbeg + wave * per );
         const int v1 = __builtin_amdgcn_readfirstlane( min( pend, v0 + per ) );
 

@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 
 POPULATION = [0, 1, 2, 3, 4, 5, 7, 8, 9, 0, 12, 13, 15, 16, 17, 20, 31, 32, 33, 48, 63, 64, 65,
               0, 0, 130]
-# 5.1 a cell, where the fused FP64 MPM P2G keeps the records of 16 particles; 3.0,
-# where the FP32 one does too and sums groups of up to four in two chains.
+# 5.1 a cell, where the fused MPM P2G keeps the records of 16 particles; 3.0, where
+# the FP32 one also sums groups of up to four in two chains.
 SPARSE = [0, 1, 2, 3, 4, 0, 0, 16, 17, 0, 0, 1, 33, 0, 0, 5]
 THIN = [0, 1, 2, 3, 4, 0, 0, 16, 17, 0, 0, 1, 0, 0, 0, 4]
 CELLS = (5, 7, 19)
