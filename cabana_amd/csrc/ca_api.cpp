@@ -794,12 +794,15 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
     // Scatters: the shape of least estimated time, (particles + node_cost *
     // window nodes) of a part times the rounds its launch takes (slots: the
     // workgroups that run at once), the last of which is partly filled.  Fitted to
-    // the 13 shapes of 31 meshes, P2G and G2P adjoint: the shape taken is 0.7 % off
-    // the fastest in the mean and 10 % at most, where the largest brick that leaves
-    // 512 of them lost up to a third (the FP64 G2P adjoint of 64^3 x 16, quadratic:
-    // 301 us with 4 x 4 x 8 cells, 317 with 6 x 6 x 8, 443 with 8 x 8 x 8).  A part
-    // is a whole brick, or an equal share of it of 1024 particles or more where
-    // there are few bricks.
+    // the 9 to 13 shapes of 40 meshes, uniform and clustered, P2G and G2P adjoint:
+    // the shape taken is 1 % off the best in the mean and 13 % at most, where the
+    // largest brick that leaves 512 of them lost up to a third (the FP64 G2P
+    // adjoint of 64^3 x 16, quadratic: 301 us with 4 x 4 x 8 cells, 317 with
+    // 6 x 6 x 8, 443 with 8 x 8 x 8).  A part is a whole brick, or an equal share
+    // of it of 1024 particles or more where there are few bricks; in a clustered
+    // cloud it is cut at 512 particles where the launch is short, at 1024
+    // otherwise (the FP32 adjoint of 64^3 x 2 98 -> 89 us with 512, the MPM P2G of
+    // 128^3 x 4 920 -> 1013 us).
     // In FP32 every part's sums are rounded as they are added to the grid (and
     // the longer chains of dense cells have their own error), so a part has 300
     // particles and 50 a cell at least (1000 at most), or the largest brick: with
@@ -834,8 +837,10 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
                       cuts *= 2.0 )
                 {
                     const double rounds = std::max( bricks * cuts / slots, 1.0 );
+                    const double idle =
+                        ( std::ceil( rounds ) - rounds ) * std::min( 1.0, 3.0 / rounds );
                     const double time = ( brick / cuts + node_cost * nodes ) *
-                                        ( 0.4 * rounds + 0.6 * std::ceil( rounds ) + 0.3 );
+                                        ( rounds + 0.6 * idle + 0.3 );
                     // Particles a part holds, as far as the FP32 rule asks for them.
                     const double held =
                         fp64 ? 0.0
@@ -848,7 +853,8 @@ bool choose_shape( TileKind kind, bool fp64, const int* slot_ng, int nslot, int 
                     best_bricks = bricks;
                     found = true;
                     double cap = 1.25 * brick / cuts;
-                    cap = cap < 1024 ? 1024 : ( cap > ( 1 << 20 ) ? ( 1 << 20 ) : cap );
+                    const int floor = rounds > 2.0 ? 1024 : 512;
+                    cap = cap < floor ? floor : ( cap > ( 1 << 20 ) ? ( 1 << 20 ) : cap );
                     sh.cap = ( (int)cap + 63 ) / 64 * 64;
                     out = sh;
                 }
