@@ -650,8 +650,8 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                     const int i0 = (int)x0;
                     const Real fr = (Real)( x0 - (double)i0 );
                     const int rel = i0 - ORDER / 2 - wlo[d];
-                    fits = fits && x0 >= 0.0 && x0 < 2147483648.0 &&
-                           (unsigned)( rel - rmin[d] ) < (unsigned)rcount[d];
+                    fits = fits & ( x0 >= 0.0 ) & ( x0 < 2147483648.0 ) &
+                           ( (unsigned)( rel - rmin[d] ) < (unsigned)rcount[d] );
                     int l = rel;
                     if constexpr ( ORDER == 2 )
                     {
@@ -707,7 +707,8 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
             // with them (fresh: 1.63 and 1.17 ms).
             int before = __shfl_up( key, 1, 64 );
             uint64_t starts = __ballot( key != before ) | 1;
-            int skey = key, rank = lane;
+            int skey = key;
+            unsigned rank = lane;
             if ( __popcll( __ballot( key < before ) ) >= SORT_DESCENTS )
             {
                 const uint32_t o = sort_lanes( (uint32_t)key << 6 | (uint32_t)lane );
@@ -717,13 +718,13 @@ __global__ __launch_bounds__( SCATTER_BLOCK, ( scatter_waves( sizeof( Real ) == 
                 starts = __ballot( skey != before ) | 1;
             }
 
+            Real* rp = rec + __mul24( rank % SUB, RS );
             static_for<64 / SUB>( [&]( auto IS ) {
                 constexpr int s0 = IS * SUB;
                 if ( s0 >= nb )
                     return;
-                if ( ( rank & ~( SUB - 1 ) ) == s0 && key >= 0 )
+                if ( rank / SUB == IS && key >= 0 )
                 {
-                    Real* rp = rec + __mul24( rank - s0, RS );
 #pragma unroll
                     for ( int n = 0; n < 4; ++n )
                     {
