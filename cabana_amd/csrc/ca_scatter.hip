@@ -23,14 +23,14 @@
 // What bounds it: instruction issue.  FP32 matrix and vector instructions do
 // not overlap on a SIMD of this chip (137 and 166 cycles of each alone take 299
 // together), so a batch of 64 particles of the MPM P2G, quadratic, FP32, costs
-// the 2930 vector and 2340 matrix cycles of its wave one after the other, and
-// waits for LDS take most of the remaining 1700.  HBM moves 2.6 GB in 1.52 ms.
+// the 3270 vector and 2340 matrix cycles of its wave one after the other, and
+// waits for LDS take most of the remaining 1750.  HBM moves 2.6 GB in 1.57 ms.
 // Against the kernel this one replaced, which sorted each task's particles in
 // LDS and added their 27 nodes by LDS atomics, spent half its time at barriers:
-//   MPM P2G, 33.6 M particles of 128^3 cells, quadratic, FP32  2.47 -> 1.52 ms
+//   MPM P2G, 33.6 M particles of 128^3 cells, quadratic, FP32  2.47 -> 1.57 ms
 //   MPM P2G, odd grid, cubic, FP64                             0.70 -> 0.36 ms
-//   mass and momentum, 8.4 M clustered particles, FP32         0.70 -> 0.46 ms
-//   MPM P2G, 7.1 M particles of 96^3 cells, linear, FP64       0.43 -> 0.39 ms
+//   mass and momentum, 8.4 M clustered particles, FP32         0.70 -> 0.45 ms
+//   MPM P2G, 7.1 M particles of 96^3 cells, linear, FP64       0.49 -> 0.37 ms
 // (linear splines in 16 x 16 products: 0.52 ms).
 #include "ca_tiles.hpp"
 

@@ -150,8 +150,9 @@ typedef struct
  * mesh's own cells.  The interpolation calls then walk particles [begin, end)
  * as cell-sorted bricks; the binning only affects speed: particles outside
  * [begin, end), and particles that moved after the binning was built, are
- * interpolated exactly like the rest (through global memory instead of the
- * brick's LDS window).  counts/offsets must still partition [begin, end).
+ * interpolated exactly like the rest.  Moved particles cost time: the scatters
+ * regroup those out of cell order, and one whose stencil leaves its brick's
+ * LDS window goes through global memory.  counts/offsets must still partition [begin, end).
  * NULL means "no ordering is known".
  * serial: 0, or a value returned by cabana_amd_new_binning_serial for this
  * build of counts/offsets.  Calls that pass the same non-zero serial (and
@@ -492,8 +493,8 @@ cabana_amd_status cabana_amd_particle_migrate(
 
 /* Calls that pass no binning (bins NULL, the drop-in shape of Cabana's p2g
  * and g2p) with spline orders 1 to 3 bin the particles by owned cell
- * themselves on the call's stream (cell keys, a stable radix sort or, up to
- * about 2^20 particles, a count by cell; in context scratch) and run the
+ * themselves on the call's stream (cell keys, a stable radix sort or, from
+ * 4097 to about 2^20 particles, a count by cell; in context scratch) and run the
  * cell-tiled kernels, reading
  * the particles in cell order through the sorted permutation; the
  * particles are not moved.  Results are those of the per-particle path up
